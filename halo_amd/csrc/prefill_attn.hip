@@ -32,6 +32,17 @@
 // tile t, which lets the matrix core and the VALU overlap within a wave.
 // Workgroups of one KV group run on one XCD (they share its L2), the ones with
 // the longest causal extent first.
+//
+// Calls whose rows give fewer workgroups than CUs leave the chip idle (512
+// rows x 32/8 heads: 64 of 256; the time is that of one workgroup's walk over
+// all keys).  There the walk is cut into n_split runs of key tiles, one
+// workgroup each, and prefill_merge_kernel folds the fp32 partials
+// (halo_prefill_splits holds the rule).  Per call, kernels only, bf16:
+//   512 rows over 8192 + 512 keys, 32/8 x 128:    238.6 us -> 90.4 us (4 splits)
+//   64 rows over 8192 + 64 keys, 32/8 x 128:      214.7 us -> 33.5 us (22)
+//   2 x 137 rows over 3000 + 137, 16/4 x 64, f16:  66.7 us -> 24.0 us (10)
+// The partials cost 2 x 4 bytes of traffic per output element and split, which
+// is why the rule stops at one workgroup per CU instead of cutting further.
 
 #include <type_traits>
 
@@ -121,6 +132,10 @@ struct PrefillParams {
   int64_t o_stride_b, o_stride_h, o_stride_t;
   int out_dtype, out_vec4;
   float* lse;  // (B, H, T_q) contiguous, or null
+  // split walk (n_split > 1): the partials of (split, unit, wave), see PfPart
+  int n_split;
+  float4* part_o;
+  float2* part_ml;
 };
 
 constexpr int kPfNW = 8;             // waves per workgroup
@@ -154,7 +169,81 @@ struct PfTile {
   bool valid;
 };
 
-template <int DT, int D>
+// Workgroup order shared by the attention and the merge launch: XCD-aware
+// (blockIdx % 8), a contiguous run of (KV group, split, workgroup) per XCD, so
+// the workgroups that read the same K/V rows share an L2; within a group the
+// workgroups with the most keys start first.
+struct PfUnit {
+  int unit, split, grp, wg;
+};
+__device__ __forceinline__ PfUnit pf_unit(const PrefillParams& P, int blk) {
+  const int n = P.n_units * P.n_split;
+  int u = blk;
+  if ((n & 7) == 0) u = (blk & 7) * (n >> 3) + (blk >> 3);
+  PfUnit r;
+  const int per = P.n_wg * P.n_split;
+  r.grp = u / per;
+  const int x = u - r.grp * per;
+  r.split = x / P.n_wg;
+  r.wg = P.n_wg - 1 - (x - r.split * P.n_wg);
+  r.unit = r.grp * P.n_wg + r.wg;
+  return r;
+}
+
+// Partial of one wave of a split unit, in the wave's own register order so
+// that every store and load is 1 KiB of consecutive bytes: piece x = 4 db + i
+// of lane l is the float4 at ((split * n_units + unit) * waves + wave) * PIECES
+// * 64 + x * 64 + l, its (m, l) pair at (...) * 32 + row.
+__device__ __forceinline__ int64_t pf_part(const PrefillParams& P, int split, int unit, int wave) {
+  return ((int64_t)split * P.n_units + unit) * kPfNW + wave;
+}
+
+// Where split `split` of n_split starts in the walk of batch row `b` (keys up
+// to `qmax`), and how many tiles it takes: lane l reads descriptor c0 + l, so
+// the whole table costs one memory round trip per 64 chunks and not one per
+// chunk.  Every lane returns the same values.
+__device__ __forceinline__ void pf_split_range(const halo_chunk_desc* descs, int n_desc, int b, int64_t qmax, int tile,
+                                               int split, int n_split, int& chunk, int& kt, int& n) {
+  const int lane = threadIdx.x & 63;
+  auto scan = [&](int c0, int& mine) {  // inclusive prefix of the tile counts of chunks [c0, c0 + 64)
+    mine = 0;
+    if (c0 + lane < n_desc) {
+      const halo_chunk_desc* d = descs + c0 + lane;
+      if (d->batch < 0 || d->batch == b) {
+        int64_t rows = d->T_c;
+        if (d->flags & HALO_CHUNK_CAUSAL) rows = min<int64_t>(rows, qmax - d->chunk_start + 1);
+        if (rows > 0) mine = (int)((rows + tile - 1) / tile);
+      }
+    }
+    int x = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int y = __shfl_up(x, off, 64);
+      if (lane >= off) x += y;
+    }
+    return x;
+  };
+  int total = 0, mine;
+  for (int c0 = 0; c0 < n_desc; c0 += 64) total += __shfl(scan(c0, mine), 63, 64);
+  const int t0 = uni((int)((int64_t)total * split / n_split));
+  n = uni((int)((int64_t)total * (split + 1) / n_split)) - t0;
+  chunk = n_desc;
+  kt = 0;
+  int base = 0;
+  for (int c0 = 0; n > 0 && c0 < n_desc; c0 += 64) {
+    const int x = base + scan(c0, mine);
+    const uint64_t past = __ballot(x > t0);
+    if (past != 0) {
+      const int at = __builtin_ctzll(past);
+      chunk = uni(c0 + at);
+      kt = uni((t0 - (__shfl(x, at, 64) - __shfl(mine, at, 64))) * tile);
+      return;
+    }
+    base = __shfl(x, 63, 64);
+  }
+}
+
+template <int DT, int D, bool SPLIT>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_attn_kernel(PrefillParams P) {
   constexpr int KS = D / 16;               // d-steps of the score MFMA
   constexpr int DB = D / 32;               // d-blocks of the output MFMA
@@ -175,13 +264,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int wave = uni(tid >> 6);
   const int qc = lane & 31, hh = lane >> 5;
 
-  // XCD-aware unit order: the units of one XCD (blockIdx % 8) are a
-  // contiguous run, so the workgroups of one KV group share an L2; within a
-  // group the workgroups with the most keys start first.
-  int unit = blockIdx.x;
-  if ((P.n_units & 7) == 0) unit = (blockIdx.x & 7) * (P.n_units >> 3) + (blockIdx.x >> 3);
-  const int grp = unit / P.n_wg;
-  const int wg = P.n_wg - 1 - unit % P.n_wg;
+  const PfUnit un = pf_unit(P, blockIdx.x);
+  const int grp = un.grp, wg = un.wg;
   const int b = grp / P.H_kv, h_kv = grp % P.H_kv;
   const int RG = P.T_q * P.rep;  // flattened rows of the group
   const int wrow0 = wg * kPfRows;
@@ -233,8 +317,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       return;
     }
   };
+  int left = 0;  // tiles from the furthest cursor to the end of this split, itself included
   auto next_tile = [&](PfTile& t) {
     if (!t.valid) return;
+    if constexpr (SPLIT) {
+      if (--left <= 0) {
+        t.valid = false;
+        return;
+      }
+    }
     t.kt += kPfBK;
     if (t.kt >= t.rows) open_chunk(t.ci + 1, t);
   };
@@ -287,7 +378,14 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   float m_run = -INFINITY, l_run = 0.f;
 
   PfTile c0, c1, c2;
-  open_chunk(0, c0);
+  if constexpr (SPLIT) {
+    int chunk, kt;
+    pf_split_range(P.descs, P.n_desc, b, wg_qmax, kPfBK, un.split, P.n_split, chunk, kt, left);
+    open_chunk(chunk, c0);
+    c0.kt = kt;
+  } else {
+    open_chunk(0, c0);
+  }
   c1 = c0;
   next_tile(c1);
   c2 = c1;
@@ -441,6 +539,17 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   // normalise and store: lane holds O^T[d][q] for MFMA rows m = 8i + 4h + j
   const float lt = half_sum(l_run);
+  if constexpr (SPLIT) {
+    const int64_t pw = pf_part(P, un.split, un.unit, wave);
+    float4* po = P.part_o + pw * (DB * 4 * 64) + lane;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        po[(db * 4 + i) * 64] = make_float4(o[db][4 * i], o[db][4 * i + 1], o[db][4 * i + 2], o[db][4 * i + 3]);
+    if (hh == 0) P.part_ml[pw * 32 + qc] = make_float2(m_run, lt);
+    return;
+  }
   if (row_ok) {
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
     const int64_t ob = (int64_t)b * P.o_stride_b + (int64_t)h * P.o_stride_h + (int64_t)pos * P.o_stride_t;
@@ -465,15 +574,135 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
+// Merge of the n_split partials of every flattened query row: one wave per
+// (unit, wave, 4 pieces), reading the partials in the order they were stored.
+// With M the largest of the row's running maxima, out = sum_s 2^(m_s - M) o_s /
+// sum_s 2^(m_s - M) l_s; a split without visible keys has m = -inf and weight 0.
+template <int D>
+__global__ void __launch_bounds__(256) prefill_merge_kernel(PrefillParams P) {
+  constexpr int PIECES = D / 8;  // float4 pieces of a lane
+  constexpr int PPW = 4;         // of which a wave of this launch merges
+  const int lane = threadIdx.x & 63;
+  const int job = uni((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int x0 = (job % (PIECES / PPW)) * PPW;
+  const int wave = (job / (PIECES / PPW)) % kPfNW;
+  const int unit = job / (PIECES / PPW) / kPfNW;
+  if (unit >= P.n_units) return;
+  const int grp = unit / P.n_wg, wg = unit - grp * P.n_wg;
+  const int b = grp / P.H_kv, h_kv = grp % P.H_kv;
+  const int qc = lane & 31, hh = lane >> 5;
+  const int r = wg * kPfRows + wave * 32 + qc;
+  if (r >= P.T_q * P.rep) return;
+  const int pos = r / P.rep;
+  const int h = h_kv * P.rep + (r - pos * P.rep);
+
+  float m = -INFINITY, l = 0.f;
+  float4 acc[PPW];
+#pragma unroll
+  for (int x = 0; x < PPW; ++x) acc[x] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int s = 0; s < P.n_split; ++s) {
+    const int64_t pw = pf_part(P, s, unit, wave);
+    const float2 ml = P.part_ml[pw * 32 + qc];
+    float4 v[PPW];
+#pragma unroll
+    for (int x = 0; x < PPW; ++x) v[x] = P.part_o[pw * (PIECES * 64) + (x0 + x) * 64 + lane];
+    const float mn = fmaxf(m, ml.x);
+    const float ms = mn == -INFINITY ? 0.f : mn;
+    const float wo = __builtin_amdgcn_exp2f(m - ms), wn = __builtin_amdgcn_exp2f(ml.x - ms);
+    m = mn;
+    l = l * wo + ml.y * wn;
+#pragma unroll
+    for (int x = 0; x < PPW; ++x) {
+      acc[x].x = __builtin_fmaf(v[x].x, wn, acc[x].x * wo);
+      acc[x].y = __builtin_fmaf(v[x].y, wn, acc[x].y * wo);
+      acc[x].z = __builtin_fmaf(v[x].z, wn, acc[x].z * wo);
+      acc[x].w = __builtin_fmaf(v[x].w, wn, acc[x].w * wo);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int64_t ob = (int64_t)b * P.o_stride_b + (int64_t)h * P.o_stride_h + (int64_t)pos * P.o_stride_t;
+#pragma unroll
+  for (int x = 0; x < PPW; ++x) {
+    const int db = (x0 + x) >> 2, mrow = 8 * ((x0 + x) & 3) + 4 * hh;
+    const int d = (mrow >> 4) * (D / 2) + 16 * db + (mrow & 15);
+    const float v4[4] = {acc[x].x * inv, acc[x].y * inv, acc[x].z * inv, acc[x].w * inv};
+    if (P.out_vec4) {
+      store_elem4(P.out, ob + d, P.out_dtype, v4);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) store_elem(P.out, ob + d + j, P.out_dtype, v4[j]);
+    }
+  }
+  if (P.lse != nullptr && hh == 0 && x0 == 0)
+    P.lse[((int64_t)b * P.H + h) * P.T_q + pos] = l > 0.f ? (m + log2f(l)) * kLn2 : -INFINITY;
+}
+
 }  // namespace halo
 
 using namespace halo;
 
-extern "C" int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
-                                 int dtype, int B, int H, int H_kv, int T_q, int D, const int64_t* q_start,
-                                 const halo_chunk_desc* descs, int n_desc, float scale,
-                                 void* out, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_t,
-                                 int out_dtype, float* lse, void* stream) {
+namespace {
+
+int64_t prefill_units(int B, int H, int H_kv, int T_q, int64_t* n_wg) {
+  const int64_t rows = (int64_t)T_q * (H / H_kv);
+  *n_wg = (rows + kPfRows - 1) / kPfRows;
+  return (int64_t)B * H_kv * *n_wg;
+}
+
+constexpr int kPfMaxSplit = 32;
+
+// bytes of one wave's partial: 32 rows x D fp32 and 32 (m, l) pairs
+int64_t prefill_part_bytes(int D) { return 32ll * D * 4 + 32 * 8; }
+
+}  // namespace
+
+// The number of key splits by a cost model of one call, in us: `rounds` of one
+// 8-wave workgroup per CU, each `mean` tiles at the measured time of a 64-key
+// tile (1.75 us at D = 128, 1.2 us at D = 64, every CU busy) plus prologue and
+// epilogue, or the longest workgroup alone; a split call adds the merge launch
+// and the partials written and read at 4 TB/s.  Against a sweep of 1 to 32
+// splits over 17 shapes (8 to 2500 rows, 0 to 16384 prior keys, 64 to 560
+// units) the choice was the fastest or within 5 % of it, but for one
+// (256 rows over 2048 keys 37.5 us for 35.6 us).
+extern "C" int halo_prefill_splits(int B, int H, int H_kv, int T_q, int D, int64_t keys, int64_t causal_keys) {
+  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || T_q <= 0 || D <= 0 || keys <= 0) return 1;
+  int64_t n_wg;
+  const int64_t units = prefill_units(B, H, H_kv, T_q, &n_wg);
+  const int cus = 256;  // one 8-wave workgroup per CU
+  const double tile_us = D == 128 ? 1.75 : 1.2, fixed_us = 4.0;
+  const double longest = (double)(keys + kPfBK - 1) / kPfBK;
+  const int64_t tri = causal_keys < T_q ? causal_keys : T_q;
+  const double mean = longest - 0.5 * (double)tri / kPfBK;
+  double best = 0;
+  int best_s = 1;
+  for (int s = 1; s <= kPfMaxSplit && s <= (int)longest; ++s) {
+    const double rounds = (double)((units * s + cus - 1) / cus);
+    const double chip = rounds * (mean / s * tile_us + fixed_us);
+    const double one = std::ceil(longest / s) * tile_us + fixed_us;
+    double us = chip > one ? chip : one;
+    if (s > 1) us += 5.0 + (double)s * (double)(units * kPfNW * prefill_part_bytes(D)) * 2.0 / 4.0e6;
+    if (s == 1 || us < best) {
+      best = us;
+      best_s = s;
+    }
+  }
+  return best_s;
+}
+
+extern "C" size_t halo_prefill_workspace_size(int B, int H, int H_kv, int T_q, int D, int n_split) {
+  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || T_q <= 0 || D <= 0 || n_split <= 1) return 0;
+  int64_t n_wg;
+  const int64_t units = prefill_units(B, H, H_kv, T_q, &n_wg);
+  return (size_t)n_split * (size_t)units * kPfNW * (size_t)prefill_part_bytes(D);
+}
+
+extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                                       int dtype, int B, int H, int H_kv, int T_q, int D, const int64_t* q_start,
+                                       const halo_chunk_desc* descs, int n_desc, float scale,
+                                       void* out, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_t,
+                                       int out_dtype, float* lse, int n_split, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
   HALO_CHECK_ARG(q && q_start && descs && out, "null pointer argument");
   HALO_CHECK_ARG(dtype == HALO_BF16 || dtype == HALO_F16, "prefill runs on bf16/fp16 MFMA: dtype must be bf16 or f16");
   HALO_CHECK_ARG(out_dtype == HALO_F32 || out_dtype == HALO_BF16 || out_dtype == HALO_F16, "bad out_dtype");
@@ -483,7 +712,12 @@ extern "C" int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_st
   HALO_CHECK_ARG(reinterpret_cast<uintptr_t>(q) % 16 == 0 && (q_stride_t * 2) % 16 == 0 && (q_stride_h * 2) % 16 == 0 &&
                      (q_stride_b * 2) % 16 == 0,
                  "q rows must be 16-byte aligned");
+  HALO_CHECK_ARG(n_split >= 1 && n_split <= kPfMaxSplit, "n_split must be in [1, 32]");
   if (T_q == 0) return HALO_OK;
+  const size_t ws_need = halo_prefill_workspace_size(B, H, H_kv, T_q, D, n_split);
+  HALO_CHECK_ARG(ws_need == 0 || (workspace != nullptr && workspace_bytes >= ws_need &&
+                                  reinterpret_cast<uintptr_t>(workspace) % 16 == 0),
+                 "workspace missing, too small or not 16-byte aligned");
   PrefillParams p;
   p.q = q;
   p.q_stride_b = q_stride_b;
@@ -495,9 +729,15 @@ extern "C" int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_st
   p.rep = H / H_kv;
   p.T_q = T_q;
   const int64_t rows = (int64_t)T_q * p.rep;
-  p.n_wg = (int)((rows + kPfRows - 1) / kPfRows);
-  const int64_t units = (int64_t)B * H_kv * p.n_wg;
-  HALO_CHECK_ARG(rows < (1ll << 31) && units < (1ll << 31), "too many query rows");
+  int64_t n_wg;
+  const int64_t units = prefill_units(B, H, H_kv, T_q, &n_wg);
+  p.n_wg = (int)n_wg;
+  HALO_CHECK_ARG(rows < (1ll << 31) && units * n_split < (1ll << 31) &&
+                     (n_split == 1 || units * kPfNW * (D / 32) < (1ll << 31)),
+                 "too many query rows");
+  p.n_split = n_split;
+  p.part_o = reinterpret_cast<float4*>(workspace);
+  p.part_ml = reinterpret_cast<float2*>(p.part_o + (n_split > 1 ? units * kPfNW * n_split * (D / 8) * 64 : 0));
   p.n_units = (int)units;
   p.q_start = q_start;
   p.descs = descs;
@@ -515,14 +755,36 @@ extern "C" int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_st
                (out_stride_h * es) % ea == 0 && (out_stride_t * es) % ea == 0;
   p.lse = lse;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(p.n_units), block(kPfNW * 64);
+  const dim3 grid((unsigned)(units * n_split)), block(kPfNW * 64);
+#define HALO_PREFILL(DTV, DV)                                                                        \
+  do {                                                                                               \
+    if (n_split > 1) hipLaunchKernelGGL((prefill_attn_kernel<DTV, DV, true>), grid, block, 0, st, p); \
+    else hipLaunchKernelGGL((prefill_attn_kernel<DTV, DV, false>), grid, block, 0, st, p);           \
+  } while (0)
   if (dtype == HALO_BF16) {
-    if (D == 128) hipLaunchKernelGGL((prefill_attn_kernel<HALO_BF16, 128>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((prefill_attn_kernel<HALO_BF16, 64>), grid, block, 0, st, p);
+    if (D == 128) HALO_PREFILL(HALO_BF16, 128);
+    else HALO_PREFILL(HALO_BF16, 64);
   } else {
-    if (D == 128) hipLaunchKernelGGL((prefill_attn_kernel<HALO_F16, 128>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((prefill_attn_kernel<HALO_F16, 64>), grid, block, 0, st, p);
+    if (D == 128) HALO_PREFILL(HALO_F16, 128);
+    else HALO_PREFILL(HALO_F16, 64);
+  }
+#undef HALO_PREFILL
+  if (n_split > 1) {
+    const int64_t jobs = units * kPfNW * (D / 8 / 4);
+    const dim3 mgrid((unsigned)((jobs + 3) / 4));
+    if (D == 128) hipLaunchKernelGGL((prefill_merge_kernel<128>), mgrid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((prefill_merge_kernel<64>), mgrid, dim3(256), 0, st, p);
   }
   HALO_CHECK_HIP(hipGetLastError());
   return HALO_OK;
+}
+
+extern "C" int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                                 int dtype, int B, int H, int H_kv, int T_q, int D, const int64_t* q_start,
+                                 const halo_chunk_desc* descs, int n_desc, float scale,
+                                 void* out, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_t,
+                                 int out_dtype, float* lse, void* stream) {
+  return halo_prefill_attn_split(q, q_stride_b, q_stride_h, q_stride_t, dtype, B, H, H_kv, T_q, D, q_start, descs,
+                                 n_desc, scale, out, out_stride_b, out_stride_h, out_stride_t, out_dtype, lse, 1,
+                                 nullptr, 0, stream);
 }

@@ -3,7 +3,8 @@
 ``prefill_attention(q, chunks)`` attends a block of query rows to a list of
 KV chunks (prior context chunks plus the query block's own K/V, the latter
 causal) and returns the output, optionally with the log-sum-exp, in one
-launch of ``halo_prefill_attn``.  fp32 queries run on the decode kernel's
+call of ``halo_prefill_attn_split``: one launch, or a few key splits and
+their merge where the query rows alone do not fill the GPU.  fp32 queries run on the decode kernel's
 fp32 path instead: the query rows of each batch row are laid out as the
 batch of one ``halo_decode_attn`` launch whose chunk descriptors repeat the
 same K/V for every such row (batch stride 0), with the causal position of
@@ -68,11 +69,15 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
         d_descs = descs_to_device(descs, q.device)
         out = torch.empty((B, H, T_q, D), device=q.device, dtype=out_dtype or q.dtype)
         lse = torch.empty((B, H, T_q), device=q.device, dtype=torch.float32) if return_lse else None
-        nat.check(L.halo_prefill_attn(
+        n_split = L.halo_prefill_splits(B, H, H_kv, T_q, D, sum(c.T for c in chunks),
+                                        sum(c.T for c in chunks if c.causal))
+        ws_bytes = L.halo_prefill_workspace_size(B, H, H_kv, T_q, D, n_split)
+        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
+        nat.check(L.halo_prefill_attn_split(
             q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), nat.dtype_code(q.dtype), B, H, H_kv, T_q, D,
             q_start.data_ptr(), d_descs.data_ptr(), len(chunks), scale,
             out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), nat.dtype_code(out.dtype),
-            nat.ptr(lse), nat.stream_ptr(stream)), "halo_prefill_attn")
+            nat.ptr(lse), n_split, nat.ptr(ws), ws_bytes, nat.stream_ptr(stream)), "halo_prefill_attn_split")
     del keep
     return (out, lse) if return_lse else out
 

@@ -262,6 +262,24 @@ int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, int
                       void* out, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_t,
                       int out_dtype, float* lse, void* stream);
 
+/*
+ * The same attention with the keys of every query block cut into n_split
+ * consecutive runs of 64-row tiles, one workgroup each, and a merge of the
+ * fp32 partials (n_split 1: halo_prefill_attn, no workspace).  For calls with
+ * too few query rows to fill the GPU.  `workspace` (16-byte aligned) holds at
+ * least halo_prefill_workspace_size bytes; halo_prefill_splits returns the
+ * n_split (1 to 32) expected to be the fastest over `keys` attended rows of
+ * which `causal_keys` are in causal chunks.
+ */
+int halo_prefill_splits(int B, int H, int H_kv, int T_q, int D, int64_t keys, int64_t causal_keys);
+size_t halo_prefill_workspace_size(int B, int H, int H_kv, int T_q, int D, int n_split);
+int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                            int dtype, int B, int H, int H_kv, int T_q, int D, const int64_t* q_start,
+                            const halo_chunk_desc* descs, int n_desc, float scale,
+                            void* out, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_t,
+                            int out_dtype, float* lse, int n_split, void* workspace, size_t workspace_bytes,
+                            void* stream);
+
 /* ---- chunk-relevance scoring ------------------------------------------- */
 
 /*
