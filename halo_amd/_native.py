@@ -107,8 +107,8 @@ _SIGNATURES = {
                               _c_void_p, _c_void_p, _c_void_p]),
     "halo_prefill_attn": (_i32, [_c_void_p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _c_void_p,
                                  _c_void_p, _i32, _f32, _c_void_p, _i64, _i64, _i64, _i32, _c_void_p, _c_void_p]),
-    "halo_prefill_splits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i64, _i64]),
-    "halo_prefill_workspace_size": (_size_t, [_i32, _i32, _i32, _i32, _i32, _i32]),
+    "halo_prefill_splits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32, _i64, _i64]),
+    "halo_prefill_workspace_size": (_size_t, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "halo_prefill_attn_split": (_i32, [_c_void_p, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _c_void_p,
                                        _c_void_p, _i32, _f32, _c_void_p, _i64, _i64, _i64, _i32, _c_void_p,
                                        _i32, _c_void_p, _size_t, _c_void_p]),

@@ -194,8 +194,9 @@ __device__ __forceinline__ PfUnit pf_unit(const PrefillParams& P, int blk) {
 // that every store and load is 1 KiB of consecutive bytes: piece x = 4 db + i
 // of lane l is the float4 at ((split * n_units + unit) * waves + wave) * PIECES
 // * 64 + x * 64 + l, its (m, l) pair at (...) * 32 + row.
+template <int NW>
 __device__ __forceinline__ int64_t pf_part(const PrefillParams& P, int split, int unit, int wave) {
-  return ((int64_t)split * P.n_units + unit) * kPfNW + wave;
+  return ((int64_t)split * P.n_units + unit) * NW + wave;
 }
 
 // Where split `split` of n_split starts in the walk of batch row `b` (keys up
@@ -240,6 +241,64 @@ __device__ __forceinline__ void pf_split_range(const halo_chunk_desc* descs, int
       return;
     }
     base = __shfl(x, 63, 64);
+  }
+}
+
+// First channel of the four that piece x = 4 db + i of lane half hh holds.
+// 16-bit kernel: MFMA row m of d-block db is channel (m / 16) D/2 + 16 db + m % 16.
+template <int D>
+struct PfRowsTr {
+  __device__ static __forceinline__ int first(int x, int hh) {
+    const int db = x >> 2, m = 8 * (x & 3) + 4 * hh;
+    return (m >> 4) * (D / 2) + 16 * db + (m & 15);
+  }
+};
+// fp32 kernel: row m of block db is channel m D/32 + db; piece x = i D/32 + g
+// holds channels 4 g .. 4 g + 3 of the 4 D/32 consecutive ones of rows 8 i + 4 hh + {0..3}.
+template <int D>
+struct PfRowsF32 {
+  __device__ static __forceinline__ int first(int x, int hh) {
+    constexpr int DB = D / 32;
+    return (8 * (x / DB) + 4 * hh) * DB + 4 * (x % DB);
+  }
+};
+
+__device__ __forceinline__ void pf_store4(const PrefillParams& P, int64_t at, const float* v4) {
+  if (P.out_vec4) {
+    store_elem4(P.out, at, P.out_dtype, v4);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) store_elem(P.out, at + j, P.out_dtype, v4[j]);
+  }
+}
+
+// The first chunk at or after `from` with rows for this (batch row, KV head) and keys up to `qmax`.
+template <int ESZ>
+__device__ __forceinline__ void pf_open_chunk(const PrefillParams& P, int b, int h_kv, int64_t qmax, int from,
+                                              PfTile& t) {
+  t.valid = false;
+  for (int c = uni(from); c < P.n_desc; ++c) {
+    const halo_chunk_desc* dp = P.descs + c;
+    const int batch = uni(dp->batch);
+    if (batch >= 0 && batch != b) continue;
+    const int causal = uni(dp->flags) & HALO_CHUNK_CAUSAL;
+    const int64_t cstart = uni64(dp->chunk_start);
+    int rows = uni(dp->T_c);
+    if (causal) rows = (int)max<int64_t>(0, min<int64_t>(rows, qmax - cstart + 1));
+    if (rows <= 0) continue;
+    const int64_t ksb = uni64(dp->k_stride_b), ksh = uni64(dp->k_stride_h);
+    const int64_t vsb = uni64(dp->v_stride_b), vsh = uni64(dp->v_stride_h);
+    t.kb = uniptr(dp->k) + ((batch < 0 ? (int64_t)b * ksb : 0) + (int64_t)h_kv * ksh) * ESZ;
+    t.vb = uniptr(dp->v) + ((batch < 0 ? (int64_t)b * vsb : 0) + (int64_t)h_kv * vsh) * ESZ;
+    t.kst = uni64(dp->k_stride_t) * ESZ;
+    t.vst = uni64(dp->v_stride_t) * ESZ;
+    t.cstart = cstart;
+    t.rows = rows;
+    t.kt = 0;
+    t.causal = causal;
+    t.ci = c;
+    t.valid = true;
+    return;
   }
 }
 
@@ -291,32 +350,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 
   // ---- the (chunk, 64-row tile) walk
-  auto open_chunk = [&](int from, PfTile& t) {
-    t.valid = false;
-    for (int c = uni(from); c < P.n_desc; ++c) {
-      const halo_chunk_desc* dp = P.descs + c;
-      const int batch = uni(dp->batch);
-      if (batch >= 0 && batch != b) continue;
-      const int causal = uni(dp->flags) & HALO_CHUNK_CAUSAL;
-      const int64_t cstart = uni64(dp->chunk_start);
-      int rows = uni(dp->T_c);
-      if (causal) rows = (int)max<int64_t>(0, min<int64_t>(rows, wg_qmax - cstart + 1));
-      if (rows <= 0) continue;
-      const int64_t ksb = uni64(dp->k_stride_b), ksh = uni64(dp->k_stride_h);
-      const int64_t vsb = uni64(dp->v_stride_b), vsh = uni64(dp->v_stride_h);
-      t.kb = uniptr(dp->k) + ((batch < 0 ? (int64_t)b * ksb : 0) + (int64_t)h_kv * ksh) * 2;
-      t.vb = uniptr(dp->v) + ((batch < 0 ? (int64_t)b * vsb : 0) + (int64_t)h_kv * vsh) * 2;
-      t.kst = uni64(dp->k_stride_t) * 2;
-      t.vst = uni64(dp->v_stride_t) * 2;
-      t.cstart = cstart;
-      t.rows = rows;
-      t.kt = 0;
-      t.causal = causal;
-      t.ci = c;
-      t.valid = true;
-      return;
-    }
-  };
+  auto open_chunk = [&](int from, PfTile& t) { pf_open_chunk<2>(P, b, h_kv, wg_qmax, from, t); };
   int left = 0;  // tiles from the furthest cursor to the end of this split, itself included
   auto next_tile = [&](PfTile& t) {
     if (!t.valid) return;
@@ -540,7 +574,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   // normalise and store: lane holds O^T[d][q] for MFMA rows m = 8i + 4h + j
   const float lt = half_sum(l_run);
   if constexpr (SPLIT) {
-    const int64_t pw = pf_part(P, un.split, un.unit, wave);
+    const int64_t pw = pf_part<kPfNW>(P, un.split, un.unit, wave);
     float4* po = P.part_o + pw * (DB * 4 * 64) + lane;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -557,18 +591,303 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int m = 8 * i + 4 * hh;
-        const int d = (m >> 4) * (D / 2) + 16 * db + (m & 15);
         float v4[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) v4[j] = o[db][4 * i + j] * inv;
-        if (P.out_vec4) {
-          store_elem4(P.out, ob + d, P.out_dtype, v4);
-        } else {
+        pf_store4(P, ob + PfRowsTr<D>::first(4 * db + i, hh), v4);
+      }
+    if (P.lse != nullptr && hh == 0)
+      P.lse[((int64_t)b * P.H + h) * P.T_q + pos] = lt > 0.f ? (m_run + log2f(lt)) * kLn2 : -INFINITY;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// fp32 queries and chunks: the same walk on v_mfma_f32_32x32x2 (fp32 products
+// and sums; error against 64 bits 3.3e-7, the VALU form had 3.3e-7).  Bound by the fp32 matrix
+// rate (148 TFLOP/s reached by a large product); the row-per-query form this
+// replaces read K/V once per query row and was planned on the host row by row.
+// 512 rows over 1536 prior + 512 keys, 16/4 heads x 64: kernels 1318 us -> 59 us
+// (attention 56 and 8-way merge 5 by themselves, 64 TFLOP/s), the call 7.2-8.0
+// ms -> 70 us.
+//
+// One workgroup of 4 waves takes 128 flattened rows, a wave 32 of them (the
+// columns); 32-key tiles (one MFMA block of keys: 64 cycles x (D/2 + D/2)
+// MFMAs per tile leave the next tile's LDS-DMA time to land) are double
+// buffered, one barrier per tile.  Step s of the score product multiplies
+// channel s (lane half 0) and D/2 + s (half 1), so a lane reads its key row in
+// 16-byte pieces; S^T's accumulator holds keys 8i + 4h + j, which are the two
+// keys of step (i, j) of the output product, so the probabilities are that
+// product's operand as they stand.  Output row m of block db is channel
+// m D/32 + db: one read per key step gives a lane its operand of every block.
+// ---------------------------------------------------------------------------
+constexpr int kPf32NW = 4;
+constexpr int kPf32Rows = kPf32NW * 32;
+constexpr int kPf32BK = 32;
+
+template <int D, bool SPLIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_attn_f32_kernel(PrefillParams P) {
+  constexpr int DB = D / 32;
+  constexpr int RB = D * 4;                       // row bytes
+  constexpr int SL = RB / 16;                     // 16-byte pieces per row
+  constexpr int TB = kPf32BK * RB;                // one K or V tile in LDS
+  constexpr int RPI = 1024 / RB;                  // rows per 1 KiB LDS-DMA instruction
+  constexpr int BPW = TB / 1024 / kPf32NW;        // 1 KiB DMA blocks per wave per tile
+  static_assert(BPW >= 1 && TB % (1024 * kPf32NW) == 0, "prefill tile shape");
+  __shared__ __attribute__((aligned(16))) char sK0[TB], sK1[TB], sV0[TB], sV1[TB];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = uni(tid >> 6);
+  const int qc = lane & 31, hh = lane >> 5;
+  const PfUnit un = pf_unit(P, blockIdx.x);
+  const int b = un.grp / P.H_kv, h_kv = un.grp % P.H_kv;
+  const int RG = P.T_q * P.rep;
+  const int wrow0 = un.wg * kPf32Rows;
+  const int64_t qs = P.q_start[b];
+  const int64_t wg_qmax = qs + (min(wrow0 + kPf32Rows, RG) - 1) / P.rep;
+  const int64_t wave_qmin = qs + min(wrow0 + wave * 32, RG - 1) / P.rep;
+  const bool active = wrow0 + wave * 32 < RG;  // a wave past the rows only stages tiles
+
+  const int r_lane = wrow0 + wave * 32 + qc;
+  const bool row_ok = r_lane < RG;
+  const int r_eff = row_ok ? r_lane : RG - 1;
+  const int pos = r_eff / P.rep;
+  const int h = h_kv * P.rep + (r_eff - pos * P.rep);
+  const int64_t qpos = qs + pos;
+
+  float qf[D / 2];  // channels hh D/2 + s
+  {
+    const float4* qrow = reinterpret_cast<const float4*>(
+        reinterpret_cast<const float*>(P.q) + (int64_t)b * P.q_stride_b + (int64_t)h * P.q_stride_h +
+        (int64_t)pos * P.q_stride_t + hh * (D / 2));
 #pragma unroll
-          for (int j = 0; j < 4; ++j) store_elem(P.out, ob + d + j, P.out_dtype, v4[j]);
+    for (int s = 0; s < D / 8; ++s) {
+      const float4 x = qrow[s];
+      qf[4 * s] = x.x;
+      qf[4 * s + 1] = x.y;
+      qf[4 * s + 2] = x.z;
+      qf[4 * s + 3] = x.w;
+    }
+  }
+
+  int left = 0;
+  auto open_chunk = [&](int from, PfTile& t) { pf_open_chunk<4>(P, b, h_kv, wg_qmax, from, t); };
+  auto next_tile = [&](PfTile& t) {
+    if (!t.valid) return;
+    if constexpr (SPLIT) {
+      if (--left <= 0) {
+        t.valid = false;
+        return;
+      }
+    }
+    t.kt += kPf32BK;
+    if (t.kt >= t.rows) open_chunk(t.ci + 1, t);
+  };
+  // K pieces are swizzled (piece ^ row % 16: the 16 rows of a b128 read pass
+  // land on distinct banks), V rows are read whole.  Rows past the chunk read
+  // as zeros (buffer range check).
+  auto issue = [&](const char* base, int64_t rst, int kt, int rows, char* st, bool is_v) {
+    const __amdgpu_buffer_rsrc_t rs = prsrc(base + (int64_t)kt * rst, (int64_t)(rows - kt) * rst);
+#pragma unroll
+    for (int j = 0; j < BPW; ++j) {
+      const int blk = wave * BPW + j;
+      const int r = blk * RPI + lane / SL, slot = lane % SL;
+      const int piece = is_v ? slot : slot ^ (r & 15);
+      const int off = (int)(r * rst) + (piece << 4);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(st + blk * 1024), 16,
+                                               off, 0, 0, 0);
+    }
+  };
+
+  pf32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o[db] = pf32x16{};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  PfTile c0, c1;
+  if constexpr (SPLIT) {
+    int chunk, kt;
+    pf_split_range(P.descs, P.n_desc, b, wg_qmax, kPf32BK, un.split, P.n_split, chunk, kt, left);
+    open_chunk(chunk, c0);
+    c0.kt = kt;
+  } else {
+    open_chunk(0, c0);
+  }
+  c1 = c0;
+  next_tile(c1);
+  if (c0.valid) {
+    issue(c0.kb, c0.kst, c0.kt, c0.rows, sK0, false);
+    issue(c0.vb, c0.vst, c0.kt, c0.rows, sV0, true);
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  auto step = [&](auto stage_c) {
+    constexpr int stage = decltype(stage_c)::value;
+    const char* const sk = stage ? sK1 : sK0;
+    const char* const sv = stage ? sV1 : sV0;
+    if (c1.valid) {  // the other stage was last read before the barrier that ended the previous tile
+      issue(c1.kb, c1.kst, c1.kt, c1.rows, stage ? sK0 : sK1, false);
+      issue(c1.vb, c1.vst, c1.kt, c1.rows, stage ? sV0 : sV1, true);
+    }
+    if (active) {
+      pf32x16 S = pf32x16{};
+      // operand reads two steps (8 MFMAs, 512 cycles) ahead, in source order:
+      // left alone the compiler reads a whole tile ahead and spills at D = 128
+      int swz = (hh * (D / 8)) ^ (qc & 15);  // D / 8 is 8 or 16 and s below it: (hh D/8 + s) ^ x = s ^ swz
+      asm volatile("" : "+v"(swz));          // one xor per read: the hoisted addresses would take D / 8 registers
+      auto kread = [&](int s) { return *reinterpret_cast<const float4*>(sk + qc * RB + ((s ^ swz) << 4)); };
+      float4 kk[2] = {kread(0), kread(1)};
+#pragma unroll
+      for (int s = 0; s < D / 8; ++s) {
+        const float4 x = kk[s & 1];
+        if (s + 2 < D / 8) kk[s & 1] = kread(s + 2);
+        S = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, qf[4 * s], S, 0, 0, 0);
+        S = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, qf[4 * s + 1], S, 0, 0, 0);
+        S = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, qf[4 * s + 2], S, 0, 0, 0);
+        S = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, qf[4 * s + 3], S, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // tile-relative number of keys this lane's row sees
+      int lim = min(c0.rows - c0.kt, kPf32BK);
+      const bool diag = c0.causal && c0.cstart + c0.kt + kPf32BK - 1 > wave_qmin;
+      if (diag) {
+        const int64_t dq = qpos - (c0.cstart + c0.kt) + 1;
+        lim = dq < (int64_t)lim ? (int)max<int64_t>(dq, 0) : lim;
+      }
+      if (diag || c0.kt + kPf32BK > c0.rows) {
+        // the sign of the scale decides which infinity weighs nothing
+        const float none = P.scale2 >= 0.f ? -INFINITY : INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) S[e] = 8 * (e >> 2) + (e & 3) + 4 * hh < lim ? S[e] : none;
+      }
+      float bm = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) bm = fmaxf(bm, S[e] * P.scale2);
+      bm = half_max(bm);
+      const float m_old = m_run;
+      m_run = bm > m_old + kPfLazyMax ? bm : m_old;
+      const float ms = m_run == -INFINITY ? 0.f : m_run;
+      if (__ballot(m_run != m_old)) {
+        const float alpha = m_run != m_old ? __builtin_amdgcn_exp2f(m_old - m_run) : 1.f;
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o[db] *= alpha;
+      }
+      float p[16];
+      float ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e], P.scale2, -ms));
+        ps[e & 3] += p[e];
+      }
+      l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+      // A row in front of the diagonal has weight 0 for the keys behind it,
+      // but 0 x inf is not 0: in a diagonal tile, values that are not finite
+      // are kept out of the product and reach the rows that see them only.
+      bool odd = false;
+      if (diag) {
+        bool bad = false;
+        for (int x = lane; x < TB / 16; x += 64) {
+          const float4 y = *reinterpret_cast<const float4*>(sv + x * 16);
+          bad |= (y.x * 0.f + y.y * 0.f) + (y.z * 0.f + y.w * 0.f) != 0.f;  // inf x 0 and NaN x 0 are NaN
+        }
+        odd = __ballot(bad) != 0;
+      }
+      // A tile's products are summed by themselves and then added to O: with O
+      // as the accumulator of every product its rounding error was 1.2 x the
+      // row-by-row form's, with one addition per tile it is below it.
+      constexpr int GB = DB == 2 ? 2 : 1;  // blocks at a time: more would spill at D = 128
+      typedef __attribute__((ext_vector_type(GB))) float vrow;
+      constexpr int VR = 8 / GB;  // rows read ahead: 8 MFMAs
+#pragma unroll
+      for (int b0 = 0; b0 < DB; b0 += GB) {
+        auto vread = [&](int e) {
+          return *reinterpret_cast<const vrow*>(sv + (8 * (e >> 2) + 4 * hh + (e & 3)) * RB + (qc * DB + b0) * 4);
+        };
+        vrow vv[VR];
+#pragma unroll
+        for (int e = 0; e < VR; ++e) vv[e] = vread(e);
+        pf32x16 t[GB];
+#pragma unroll
+        for (int g = 0; g < GB; ++g) t[g] = pf32x16{};
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const vrow v = vv[e % VR];
+          if (e + VR < 16) vv[e % VR] = vread(e + VR);
+#pragma unroll
+          for (int g = 0; g < GB; ++g) {
+            const float x = odd && !(fabsf(v[g]) < INFINITY) ? 0.f : v[g];
+            t[g] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, p[e], t[g], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int g = 0; g < GB; ++g) o[b0 + g] += t[g];
+      }
+      if (odd) {
+        // how many of +inf (or NaN), then of -inf (or NaN), each row sees in each channel
+#pragma unroll
+        for (int x = 0; x < 2 * DB; ++x) {
+          const float inf = x & 1 ? -INFINITY : INFINITY;
+          pf32x16 n = pf32x16{};
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float v = *reinterpret_cast<const float*>(sv + (8 * (e >> 2) + 4 * hh + (e & 3)) * RB +
+                                                            (qc * DB + (x >> 1)) * 4);
+            const float sees = 8 * (e >> 2) + (e & 3) + 4 * hh < lim ? 1.f : 0.f;
+            n = __builtin_amdgcn_mfma_f32_32x32x2f32(v == inf || v != v ? 1.f : 0.f, sees, n, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[x >> 1][e] += n[e] > 0.f ? inf : 0.f;
         }
       }
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the next tile have landed
+    __syncthreads();                // every wave's have; this tile's stage is free
+    c0 = c1;
+    next_tile(c1);
+  };
+  while (c0.valid) {
+    step(std::integral_constant<int, 0>());
+    if (!c0.valid) break;
+    step(std::integral_constant<int, 1>());
+  }
+
+  if (!active) return;
+  // rows m = 8i + 4h + {0..3} are 4 DB consecutive channels: DB float4s
+  const float lt = half_sum(l_run);
+  float4 piece[4 * DB];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int g = 0; g < DB; ++g) {
+      float x[4];
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const int c = 4 * g + y;  // channel within the run: (j, db) = (c / DB, c % DB)
+        x[y] = o[c % DB][4 * i + c / DB];
+      }
+      piece[i * DB + g] = make_float4(x[0], x[1], x[2], x[3]);
+    }
+  if constexpr (SPLIT) {
+    const int64_t pw = pf_part<kPf32NW>(P, un.split, un.unit, wave);
+    float4* po = P.part_o + pw * (DB * 4 * 64) + lane;
+#pragma unroll
+    for (int x = 0; x < 4 * DB; ++x) po[x * 64] = piece[x];
+    if (hh == 0) P.part_ml[pw * 32 + qc] = make_float2(m_run, lt);
+    return;
+  }
+  if (row_ok) {
+    const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    const int64_t ob = (int64_t)b * P.o_stride_b + (int64_t)h * P.o_stride_h + (int64_t)pos * P.o_stride_t;
+#pragma unroll
+    for (int x = 0; x < 4 * DB; ++x) {
+      const float v4[4] = {piece[x].x * inv, piece[x].y * inv, piece[x].z * inv, piece[x].w * inv};
+      pf_store4(P, ob + PfRowsF32<D>::first(x, hh), v4);
+    }
     if (P.lse != nullptr && hh == 0)
       P.lse[((int64_t)b * P.H + h) * P.T_q + pos] = lt > 0.f ? (m_run + log2f(lt)) * kLn2 : -INFINITY;
   }
@@ -578,20 +897,21 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 // (unit, wave, 4 pieces), reading the partials in the order they were stored.
 // With M the largest of the row's running maxima, out = sum_s 2^(m_s - M) o_s /
 // sum_s 2^(m_s - M) l_s; a split without visible keys has m = -inf and weight 0.
-template <int D>
+// NW waves per workgroup of the attention launch, PM the placement of its output rows.
+template <int D, int NW, class PM>
 __global__ void __launch_bounds__(256) prefill_merge_kernel(PrefillParams P) {
   constexpr int PIECES = D / 8;  // float4 pieces of a lane
   constexpr int PPW = 4;         // of which a wave of this launch merges
   const int lane = threadIdx.x & 63;
   const int job = uni((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
   const int x0 = (job % (PIECES / PPW)) * PPW;
-  const int wave = (job / (PIECES / PPW)) % kPfNW;
-  const int unit = job / (PIECES / PPW) / kPfNW;
+  const int wave = (job / (PIECES / PPW)) % NW;
+  const int unit = job / (PIECES / PPW) / NW;
   if (unit >= P.n_units) return;
   const int grp = unit / P.n_wg, wg = unit - grp * P.n_wg;
   const int b = grp / P.H_kv, h_kv = grp % P.H_kv;
   const int qc = lane & 31, hh = lane >> 5;
-  const int r = wg * kPfRows + wave * 32 + qc;
+  const int r = (wg * NW + wave) * 32 + qc;
   if (r >= P.T_q * P.rep) return;
   const int pos = r / P.rep;
   const int h = h_kv * P.rep + (r - pos * P.rep);
@@ -602,7 +922,7 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(PrefillParams P) {
   for (int x = 0; x < PPW; ++x) acc[x] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 4
   for (int s = 0; s < P.n_split; ++s) {
-    const int64_t pw = pf_part(P, s, unit, wave);
+    const int64_t pw = pf_part<NW>(P, s, unit, wave);
     const float2 ml = P.part_ml[pw * 32 + qc];
     float4 v[PPW];
 #pragma unroll
@@ -624,15 +944,9 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(PrefillParams P) {
   const int64_t ob = (int64_t)b * P.o_stride_b + (int64_t)h * P.o_stride_h + (int64_t)pos * P.o_stride_t;
 #pragma unroll
   for (int x = 0; x < PPW; ++x) {
-    const int db = (x0 + x) >> 2, mrow = 8 * ((x0 + x) & 3) + 4 * hh;
-    const int d = (mrow >> 4) * (D / 2) + 16 * db + (mrow & 15);
+    const int d = PM::first(x0 + x, hh);
     const float v4[4] = {acc[x].x * inv, acc[x].y * inv, acc[x].z * inv, acc[x].w * inv};
-    if (P.out_vec4) {
-      store_elem4(P.out, ob + d, P.out_dtype, v4);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) store_elem(P.out, ob + d + j, P.out_dtype, v4[j]);
-    }
+    pf_store4(P, ob + d, v4);
   }
   if (P.lse != nullptr && hh == 0 && x0 == 0)
     P.lse[((int64_t)b * P.H + h) * P.T_q + pos] = l > 0.f ? (m + log2f(l)) * kLn2 : -INFINITY;
@@ -644,9 +958,10 @@ using namespace halo;
 
 namespace {
 
-int64_t prefill_units(int B, int H, int H_kv, int T_q, int64_t* n_wg) {
+int64_t prefill_units(int dtype, int B, int H, int H_kv, int T_q, int64_t* n_wg) {
   const int64_t rows = (int64_t)T_q * (H / H_kv);
-  *n_wg = (rows + kPfRows - 1) / kPfRows;
+  const int per = dtype == HALO_F32 ? kPf32Rows : kPfRows;
+  *n_wg = (rows + per - 1) / per;
   return (int64_t)B * H_kv * *n_wg;
 }
 
@@ -664,24 +979,29 @@ int64_t prefill_part_bytes(int D) { return 32ll * D * 4 + 32 * 8; }
 // and the partials written and read at 4 TB/s.  Against a sweep of 1 to 32
 // splits over 17 shapes (8 to 2500 rows, 0 to 16384 prior keys, 64 to 560
 // units) the choice was the fastest or within 5 % of it, but for one
-// (256 rows over 2048 keys 37.5 us for 35.6 us).
-extern "C" int halo_prefill_splits(int B, int H, int H_kv, int T_q, int D, int64_t keys, int64_t causal_keys) {
+// (256 rows over 2048 keys 37.5 us for 35.6 us).  fp32: 32-key tiles, 3.1 and
+// 5.5 us with one 4-wave workgroup on a CU, 4.4 and 9.2 us each with two.
+extern "C" int halo_prefill_splits(int dtype, int B, int H, int H_kv, int T_q, int D, int64_t keys, int64_t causal_keys) {
   if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || T_q <= 0 || D <= 0 || keys <= 0) return 1;
   int64_t n_wg;
-  const int64_t units = prefill_units(B, H, H_kv, T_q, &n_wg);
-  const int cus = 256;  // one 8-wave workgroup per CU
-  const double tile_us = D == 128 ? 1.75 : 1.2, fixed_us = 4.0;
-  const double longest = (double)(keys + kPfBK - 1) / kPfBK;
+  const int64_t units = prefill_units(dtype, B, H, H_kv, T_q, &n_wg);
+  const bool f32 = dtype == HALO_F32;
+  const int bk = f32 ? kPf32BK : kPfBK, nw = f32 ? kPf32NW : kPfNW;
+  const double fixed_us = 4.0;
+  const double longest = (double)(keys + bk - 1) / bk;
   const int64_t tri = causal_keys < T_q ? causal_keys : T_q;
-  const double mean = longest - 0.5 * (double)tri / kPfBK;
+  const double mean = longest - 0.5 * (double)tri / bk;
   double best = 0;
   int best_s = 1;
   for (int s = 1; s <= kPfMaxSplit && s <= (int)longest; ++s) {
-    const double rounds = (double)((units * s + cus - 1) / cus);
+    const bool pairs = f32 && units * s > 256;  // fp32: two 4-wave workgroups per CU
+    const int slots = pairs ? 512 : 256;
+    const double tile_us = f32 ? (pairs ? (D == 128 ? 9.2 : 4.4) : (D == 128 ? 5.5 : 3.1)) : (D == 128 ? 1.75 : 1.2);
+    const double rounds = (double)((units * s + slots - 1) / slots);
     const double chip = rounds * (mean / s * tile_us + fixed_us);
     const double one = std::ceil(longest / s) * tile_us + fixed_us;
     double us = chip > one ? chip : one;
-    if (s > 1) us += 5.0 + (double)s * (double)(units * kPfNW * prefill_part_bytes(D)) * 2.0 / 4.0e6;
+    if (s > 1) us += 5.0 + (double)s * (double)(units * nw * prefill_part_bytes(D)) * 2.0 / 4.0e6;
     if (s == 1 || us < best) {
       best = us;
       best_s = s;
@@ -690,11 +1010,12 @@ extern "C" int halo_prefill_splits(int B, int H, int H_kv, int T_q, int D, int64
   return best_s;
 }
 
-extern "C" size_t halo_prefill_workspace_size(int B, int H, int H_kv, int T_q, int D, int n_split) {
+extern "C" size_t halo_prefill_workspace_size(int dtype, int B, int H, int H_kv, int T_q, int D, int n_split) {
   if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || T_q <= 0 || D <= 0 || n_split <= 1) return 0;
   int64_t n_wg;
-  const int64_t units = prefill_units(B, H, H_kv, T_q, &n_wg);
-  return (size_t)n_split * (size_t)units * kPfNW * (size_t)prefill_part_bytes(D);
+  const int64_t units = prefill_units(dtype, B, H, H_kv, T_q, &n_wg);
+  const int nw = dtype == HALO_F32 ? kPf32NW : kPfNW;
+  return (size_t)n_split * (size_t)units * nw * (size_t)prefill_part_bytes(D);
 }
 
 extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -704,17 +1025,18 @@ extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_
                                        int out_dtype, float* lse, int n_split, void* workspace,
                                        size_t workspace_bytes, void* stream) {
   HALO_CHECK_ARG(q && q_start && descs && out, "null pointer argument");
-  HALO_CHECK_ARG(dtype == HALO_BF16 || dtype == HALO_F16, "prefill runs on bf16/fp16 MFMA: dtype must be bf16 or f16");
+  HALO_CHECK_ARG(dtype == HALO_BF16 || dtype == HALO_F16 || dtype == HALO_F32, "dtype must be bf16, f16 or f32");
   HALO_CHECK_ARG(out_dtype == HALO_F32 || out_dtype == HALO_BF16 || out_dtype == HALO_F16, "bad out_dtype");
   HALO_CHECK_ARG(B > 0 && H > 0 && H_kv > 0 && H % H_kv == 0 && T_q >= 0, "need H % H_kv == 0 and positive sizes");
   HALO_CHECK_ARG(D == 64 || D == 128, "head_dim must be 64 or 128");
   HALO_CHECK_ARG(n_desc >= 0, "bad chunk count");
-  HALO_CHECK_ARG(reinterpret_cast<uintptr_t>(q) % 16 == 0 && (q_stride_t * 2) % 16 == 0 && (q_stride_h * 2) % 16 == 0 &&
-                     (q_stride_b * 2) % 16 == 0,
+  const int64_t esz = elem_size(dtype);
+  HALO_CHECK_ARG(reinterpret_cast<uintptr_t>(q) % 16 == 0 && (q_stride_t * esz) % 16 == 0 &&
+                     (q_stride_h * esz) % 16 == 0 && (q_stride_b * esz) % 16 == 0,
                  "q rows must be 16-byte aligned");
   HALO_CHECK_ARG(n_split >= 1 && n_split <= kPfMaxSplit, "n_split must be in [1, 32]");
   if (T_q == 0) return HALO_OK;
-  const size_t ws_need = halo_prefill_workspace_size(B, H, H_kv, T_q, D, n_split);
+  const size_t ws_need = halo_prefill_workspace_size(dtype, B, H, H_kv, T_q, D, n_split);
   HALO_CHECK_ARG(ws_need == 0 || (workspace != nullptr && workspace_bytes >= ws_need &&
                                   reinterpret_cast<uintptr_t>(workspace) % 16 == 0),
                  "workspace missing, too small or not 16-byte aligned");
@@ -730,19 +1052,23 @@ extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_
   p.T_q = T_q;
   const int64_t rows = (int64_t)T_q * p.rep;
   int64_t n_wg;
-  const int64_t units = prefill_units(B, H, H_kv, T_q, &n_wg);
+  const int64_t units = prefill_units(dtype, B, H, H_kv, T_q, &n_wg);
+  const int nw = dtype == HALO_F32 ? kPf32NW : kPfNW;
   p.n_wg = (int)n_wg;
   HALO_CHECK_ARG(rows < (1ll << 31) && units * n_split < (1ll << 31) &&
-                     (n_split == 1 || units * kPfNW * (D / 32) < (1ll << 31)),
+                     (n_split == 1 || units * nw * (D / 32) < (1ll << 31)),
                  "too many query rows");
   p.n_split = n_split;
   p.part_o = reinterpret_cast<float4*>(workspace);
-  p.part_ml = reinterpret_cast<float2*>(p.part_o + (n_split > 1 ? units * kPfNW * n_split * (D / 8) * 64 : 0));
+  p.part_ml = reinterpret_cast<float2*>(p.part_o + (n_split > 1 ? units * nw * n_split * (D / 8) * 64 : 0));
   p.n_units = (int)units;
   p.q_start = q_start;
   p.descs = descs;
   p.n_desc = n_desc;
   p.scale2 = (float)((double)scale * 1.4426950408889634);
+  // a masked score is an infinity times the scale: a zero scale would make it NaN,
+  // and the smallest normal number leaves every finite score at 2^0 all the same
+  if (dtype == HALO_F32 && p.scale2 == 0.f) p.scale2 = 1.17549435e-38f;
   p.out = out;
   p.o_stride_b = out_stride_b;
   p.o_stride_h = out_stride_h;
@@ -755,13 +1081,22 @@ extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_
                (out_stride_h * es) % ea == 0 && (out_stride_t * es) % ea == 0;
   p.lse = lse;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)(units * n_split)), block(kPfNW * 64);
+  const dim3 grid((unsigned)(units * n_split)), block(nw * 64);
+  if (dtype == HALO_F32) {
+    if (n_split > 1) {
+      if (D == 128) hipLaunchKernelGGL((prefill_attn_f32_kernel<128, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((prefill_attn_f32_kernel<64, true>), grid, block, 0, st, p);
+    } else {
+      if (D == 128) hipLaunchKernelGGL((prefill_attn_f32_kernel<128, false>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((prefill_attn_f32_kernel<64, false>), grid, block, 0, st, p);
+    }
+  }
 #define HALO_PREFILL(DTV, DV)                                                                        \
   do {                                                                                               \
     if (n_split > 1) hipLaunchKernelGGL((prefill_attn_kernel<DTV, DV, true>), grid, block, 0, st, p); \
     else hipLaunchKernelGGL((prefill_attn_kernel<DTV, DV, false>), grid, block, 0, st, p);           \
   } while (0)
-  if (dtype == HALO_BF16) {
+  else if (dtype == HALO_BF16) {
     if (D == 128) HALO_PREFILL(HALO_BF16, 128);
     else HALO_PREFILL(HALO_BF16, 64);
   } else {
@@ -770,10 +1105,18 @@ extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_
   }
 #undef HALO_PREFILL
   if (n_split > 1) {
-    const int64_t jobs = units * kPfNW * (D / 8 / 4);
+    const int64_t jobs = units * nw * (D / 8 / 4);
     const dim3 mgrid((unsigned)((jobs + 3) / 4));
-    if (D == 128) hipLaunchKernelGGL((prefill_merge_kernel<128>), mgrid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((prefill_merge_kernel<64>), mgrid, dim3(256), 0, st, p);
+#define HALO_MERGE(DV)                                                                                             \
+  do {                                                                                                             \
+    if (dtype == HALO_F32)                                                                                         \
+      hipLaunchKernelGGL((prefill_merge_kernel<DV, kPf32NW, PfRowsF32<DV>>), mgrid, dim3(256), 0, st, p);          \
+    else                                                                                                           \
+      hipLaunchKernelGGL((prefill_merge_kernel<DV, kPfNW, PfRowsTr<DV>>), mgrid, dim3(256), 0, st, p);             \
+  } while (0)
+    if (D == 128) HALO_MERGE(128);
+    else HALO_MERGE(64);
+#undef HALO_MERGE
   }
   HALO_CHECK_HIP(hipGetLastError());
   return HALO_OK;
@@ -784,6 +1127,7 @@ extern "C" int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_st
                                  const halo_chunk_desc* descs, int n_desc, float scale,
                                  void* out, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_t,
                                  int out_dtype, float* lse, void* stream) {
+  HALO_CHECK_ARG(dtype == HALO_BF16 || dtype == HALO_F16, "prefill runs on bf16/fp16 MFMA: dtype must be bf16 or f16");
   return halo_prefill_attn_split(q, q_stride_b, q_stride_h, q_stride_t, dtype, B, H, H_kv, T_q, D, q_start, descs,
                                  n_desc, scale, out, out_stride_b, out_stride_h, out_stride_t, out_dtype, lse, 1,
                                  nullptr, 0, stream);

@@ -1,16 +1,16 @@
-"""Chunked causal prefill attention on bf16/fp16 MFMA.
+"""Chunked causal prefill attention on MFMA (bf16, fp16, fp32).
 
 ``prefill_attention(q, chunks)`` attends a block of query rows to a list of
 KV chunks (prior context chunks plus the query block's own K/V, the latter
 causal) and returns the output, optionally with the log-sum-exp, in one
 call of ``halo_prefill_attn_split``: one launch, or a few key splits and
-their merge where the query rows alone do not fill the GPU.  fp32 queries run on the decode kernel's
-fp32 path instead: the query rows of each batch row are laid out as the
-batch of one ``halo_decode_attn`` launch whose chunk descriptors repeat the
-same K/V for every such row (batch stride 0), with the causal position of
-row i at q_start + i.  That path reads K/V once per query row; it exists
-for fp32 models (the reference computes every T_q in fp32,
-halo/kv_cache_chunked.py:241-276), not for throughput.
+their merge where the query rows alone do not fill the GPU.  fp32 queries
+(the reference computes every T_q in fp32, halo/kv_cache_chunked.py:241-276)
+take the fp32 matrix instructions.  fp32 calls whose chunks that kernel does
+not read (``_f32_direct``) run on the decode kernel: the query rows of each
+batch row are the batch of one ``halo_decode_attn`` launch whose chunk
+descriptors repeat the same K/V for every such row (batch stride 0), with the
+causal position of row i at q_start + i; it reads K/V once per query row.
 
 Reference: the chunked prefill path of HALOCacheChunked.compute_attention
 (halo/kv_cache_chunked.py:864-964), which runs _chunk_attention per chunk and
@@ -32,7 +32,7 @@ from .decode import ChunkRef, _to_device, descs_to_device, pack_descs
 def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Optional[float] = None,
                       q_start=None, out_dtype: Optional[torch.dtype] = None, return_lse: bool = False,
                       stream=None):
-    """q (B, H, T_q, D) bf16/fp16; chunks (B, H_kv, T_c, D) of the same dtype.
+    """q (B, H, T_q, D) bf16, fp16 or fp32; chunks (B, H_kv, T_c, D) of the same dtype.
     Returns out (B, H, T_q, D) in ``out_dtype`` (default q.dtype) and, with
     ``return_lse``, lse (B, H, T_q) fp32."""
     L = nat.lib()
@@ -41,16 +41,17 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
     B, H, T_q, D = q.shape
     if not chunks:
         raise AssertionError("no chunks to attend")
-    if q.dtype == torch.float32:
+    if q.dtype == torch.float32 and not _f32_direct(q, chunks):
         return _prefill_fp32_rows(q, chunks, scale=scale, q_start=q_start, out_dtype=out_dtype,
                                   return_lse=return_lse, stream=stream)
-    if q.dtype not in (torch.bfloat16, torch.float16):
-        raise AssertionError(f"prefill runs on bf16/fp16 MFMA or the fp32 decode path; got {q.dtype}")
+    if q.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+        raise AssertionError(f"prefill runs on bf16, fp16 or fp32; got {q.dtype}")
     H_kv = chunks[0].k.shape[-3]
     if H % H_kv:
         raise AssertionError(f"head count mismatch: q has {H}, kv has {H_kv}")
-    if q.stride(-1) != 1 or (q.stride(-2) * 2) % 16 or q.data_ptr() % 16:
-        q = q.contiguous()
+    q = _aligned_q(q)
+    qs_b, qs_h, qs_t = (st if n > 1 else 0 for st, n in zip(q.stride()[:3], q.shape)) if q.dtype == torch.float32 \
+        else q.stride()[:3]
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     if q_start is None:
         q_start = sum(c.T for c in chunks) - T_q
@@ -65,21 +66,51 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
             q_start = torch.full((B,), int(q_start), dtype=torch.int64, device=q.device)
         elif q_start.device.type != "cuda":
             q_start = _to_device(q_start.to(torch.int64).reshape(-1).expand(B).numpy(), q.device)
+        if q.dtype == torch.float32 and q_start.numel() == 1:
+            q_start = q_start.reshape(1).expand(B)
         q_start = q_start.to(device=q.device, dtype=torch.int64).reshape(B).contiguous()
         d_descs = descs_to_device(descs, q.device)
         out = torch.empty((B, H, T_q, D), device=q.device, dtype=out_dtype or q.dtype)
         lse = torch.empty((B, H, T_q), device=q.device, dtype=torch.float32) if return_lse else None
-        n_split = L.halo_prefill_splits(B, H, H_kv, T_q, D, sum(c.T for c in chunks),
+        dt = nat.dtype_code(q.dtype)
+        n_split = L.halo_prefill_splits(dt, B, H, H_kv, T_q, D, sum(c.T for c in chunks),
                                         sum(c.T for c in chunks if c.causal))
-        ws_bytes = L.halo_prefill_workspace_size(B, H, H_kv, T_q, D, n_split)
+        ws_bytes = L.halo_prefill_workspace_size(dt, B, H, H_kv, T_q, D, n_split)
         ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
         nat.check(L.halo_prefill_attn_split(
-            q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), nat.dtype_code(q.dtype), B, H, H_kv, T_q, D,
+            q.data_ptr(), qs_b, qs_h, qs_t, dt, B, H, H_kv, T_q, D,
             q_start.data_ptr(), d_descs.data_ptr(), len(chunks), scale,
             out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), nat.dtype_code(out.dtype),
             nat.ptr(lse), n_split, nat.ptr(ws), ws_bytes, nat.stream_ptr(stream)), "halo_prefill_attn_split")
     del keep
     return (out, lse) if return_lse else out
+
+
+def _aligned_q(q: torch.Tensor) -> torch.Tensor:
+    if q.dtype != torch.float32:
+        return q.contiguous() if q.stride(-1) != 1 or (q.stride(-2) * 2) % 16 or q.data_ptr() % 16 else q
+    odd = q.stride(-1) != 1 or q.data_ptr() % 16 or any(n > 1 and st % 4 for st, n in zip(q.stride()[:3], q.shape))
+    return q.clone(memory_format=torch.contiguous_format) if odd else q
+
+
+def _f32_direct(q: torch.Tensor, chunks: Sequence[ChunkRef]) -> bool:
+    """Whether the fp32 MFMA kernel takes the call: head dim 64 or 128 and
+    chunks of the batch whose rows and heads are 16-byte aligned and do not
+    overlap, with row strides that a tile's buffer offsets can hold.  The
+    decode kernel's row-by-row form keeps the others, and their errors."""
+    B, H, T_q, D = q.shape
+    if B == 0 or T_q == 0 or D not in (64, 128) or not q.is_cuda:
+        return False
+    for c in chunks:
+        for t in (getattr(c, "k", None), getattr(c, "v", None)):
+            if t is None or t.dim() != 4 or t.shape[0] != B or t.shape[-1] != D or t.dtype != torch.float32:
+                return False
+            if getattr(c, "batch", -1) >= 0 or t.stride(-1) != 1 or t.data_ptr() % 16:
+                return False
+            sb, sh, st = t.stride()[:3]
+            if (t.shape[0] > 1 and sb % 4) or (t.shape[1] > 1 and sh % 4) or st % 4 or not D <= st < 1 << 22:
+                return False
+    return True
 
 
 def _prefill_fp32_rows(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale, q_start, out_dtype,

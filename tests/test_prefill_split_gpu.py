@@ -11,9 +11,9 @@ import torch
 from oracle import attention as A
 from oracle.inputs import round_to
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 
-DT = {"bfloat16": torch.bfloat16, "float16": torch.float16}
+DT = {"bfloat16": torch.bfloat16, "float16": torch.float16, "float32": torch.float32}
 
 
 def _split(q, chunks, n_split, *, q_start, out_dtype=torch.float32):
@@ -27,7 +27,7 @@ def _split(q, chunks, n_split, *, q_start, out_dtype=torch.float32):
     qs = torch.full((B,), q_start, device=q.device, dtype=torch.int64)
     out = torch.full((B, H, T_q, D), float("nan"), device=q.device, dtype=out_dtype)
     lse = torch.full((B, H, T_q), float("nan"), device=q.device)
-    nb = L.halo_prefill_workspace_size(B, H, H_kv, T_q, D, n_split)
+    nb = L.halo_prefill_workspace_size(nat.dtype_code(q.dtype), B, H, H_kv, T_q, D, n_split)
     ws = torch.full((max(nb, 16),), 0xFF, device=q.device, dtype=torch.uint8)
     nat.check(L.halo_prefill_attn_split(
         q.data_ptr(), *q.stride()[:3], nat.dtype_code(q.dtype), B, H, H_kv, T_q, D, qs.data_ptr(), dd.data_ptr(),
@@ -37,13 +37,17 @@ def _split(q, chunks, n_split, *, q_start, out_dtype=torch.float32):
     return out.cpu().numpy(), lse.cpu().numpy()
 
 
+@gpu
 @pytest.mark.parametrize("dtype,B,H,H_kv,D,T_prior,T_q,chunk", [
     ("bfloat16", 1, 8, 2, 128, 384, 130, 128),   # a second, nearly empty row block
     ("float16", 2, 7, 1, 64, 130, 45, 64),       # rep 7, ragged chunk ends
     ("bfloat16", 1, 4, 4, 128, 0, 65, 64),       # self chunk only: the first rows see one tile
     ("float16", 1, 4, 1, 64, 1340, 8, 20),       # 68 chunks: the table scan takes a second batch of 64
+    ("float32", 1, 8, 2, 128, 384, 33, 128),     # 132 rows: a workgroup with one live wave
+    ("float32", 2, 7, 1, 64, 130, 45, 64),
+    ("float32", 1, 4, 1, 64, 1340, 8, 20),
 ])
-@pytest.mark.parametrize("n_split", [2, 3, 32])
+@pytest.mark.parametrize("n_split", [1, 2, 3, 32])
 def test_split_matches_closed_form(dev, dtype, B, H, H_kv, D, T_prior, T_q, chunk, n_split):
     from halo_amd.decode import ChunkRef
     rng = np.random.default_rng(17)
@@ -56,10 +60,12 @@ def test_split_matches_closed_form(dev, dtype, B, H, H_kv, D, T_prior, T_q, chun
     out, lse = _split(qg, chunks, n_split, q_start=T_prior)
     want, wl = A.prefill_f64(q, k, v, scale=1 / math.sqrt(D), q_start=T_prior)
     # the probabilities are rounded to the 16-bit type in front of the second product
-    assert np.abs(out - want).max() <= (2e-2 if dtype == "bfloat16" else 3e-3)
+    # (2^-9 and 2^-12 relative, of outputs below 4); fp32: sums of at most 1400 products of 2^-24
+    assert np.abs(out - want).max() <= {"bfloat16": 2e-2, "float16": 3e-3, "float32": 1e-5}[dtype]
     assert np.abs(lse - wl).max() <= 1e-5 * max(1.0, np.abs(wl).max())
 
 
+@gpu
 @pytest.mark.parametrize("n_split", [1, 4])
 def test_split_rows_without_keys(dev, n_split):
     """Rows in front of every causal key, and a chunk of another batch row:
@@ -77,15 +83,58 @@ def test_split_rows_without_keys(dev, n_split):
     assert np.abs(lse[1:, :, 40:] - wl).max() <= 1e-4
 
 
+@gpu
+@pytest.mark.parametrize("T_q,prior,D", [(1, 0, 64), (31, 1, 128), (40, 65, 64), (200, 300, 64)])
+@pytest.mark.parametrize("scale", [0.3, 0.0, -0.2])
+def test_fp32_call(dev, T_q, prior, D, scale):
+    """The public fp32 call: strided q, a head group that is no power of two,
+    values behind the diagonal that are not finite, any sign of the scale."""
+    from halo_amd.decode import ChunkRef
+    from halo_amd.prefill import _f32_direct, prefill_attention
+    rng = np.random.default_rng(T_q)
+    H, H_kv, T = 6, 2, prior + T_q
+    q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((1, T_q, H, D), (1, H_kv, T, D), (1, H_kv, T, D)))
+    qt = torch.from_numpy(q).to(dev).transpose(1, 2)
+    kt, vt = torch.from_numpy(k).to(dev), torch.from_numpy(v).to(dev)
+    chunks = [ChunkRef(kt[:, :, :prior], vt[:, :, :prior], 0, False)] if prior else []
+    chunks.append(ChunkRef(kt[:, :, prior:], vt[:, :, prior:], prior, True))
+    assert _f32_direct(qt, chunks)
+    out, lse = prefill_attention(qt, chunks, scale=scale, return_lse=True)
+    want, wl = A.prefill_f64(q.transpose(0, 2, 1, 3), k, v, scale=scale, q_start=prior)
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5
+    assert np.abs(lse.cpu().numpy() - wl).max() <= 1e-5 * max(1.0, np.abs(wl).max())
+    vt[:, 0, T - 1, 3], vt[:, 1, T - 1, 5], kt[:, 0, T - 1, 0] = float("inf"), float("nan"), float("nan")
+    out2 = prefill_attention(qt, chunks, scale=scale)
+    assert torch.equal(out2[:, :, :-1], out[:, :, :-1])  # only the last row sees the last key
+    assert out2[:, :3, -1, 3].isnan().all() and out2[:, 3:, -1, 5].isnan().all()
+    assert torch.equal(out2[:, 3:, -1, :5], out[:, 3:, -1, :5])
+
+
+def test_fp32_route():
+    """Chunks that the matrix kernel does not read stay on the row-by-row form."""
+    from halo_amd.decode import ChunkRef
+    from halo_amd.prefill import _f32_direct
+
+    class Q:  # a device query of this shape
+        is_cuda, shape = True, (1, 4, 8, 64)
+    k = torch.zeros((1, 2, 32, 64))
+    assert _f32_direct(Q, [ChunkRef(k, k, 0, True)])
+    for odd in (k[0], k.double(), torch.zeros((1, 2, 32, 66))[..., :64], k[:, :, :1].expand(1, 2, 32, 64),
+                torch.zeros((2, 2, 32, 64)), torch.zeros(4098)[2:].view(1, 1, 64, 64)):
+        assert not _f32_direct(Q, [ChunkRef(odd, odd, 0, True)])
+    assert not _f32_direct(Q, [ChunkRef(k[0], k[0], 0, True, batch=0)])
+
+
+@gpu
 def test_split_choice():
     """One pass where the query rows fill the GPU, and no more passes than
     64-row tiles or than the limit."""
     from halo_amd import _native as nat
     L = nat.lib()
-    assert L.halo_prefill_splits(1, 32, 8, 4096, 128, 32768, 4096) == 1
-    assert L.halo_prefill_splits(1, 32, 8, 512, 128, 60, 60) == 1
+    assert L.halo_prefill_splits(nat.BF16, 1, 32, 8, 4096, 128, 32768, 4096) == 1
+    assert L.halo_prefill_splits(nat.BF16, 1, 32, 8, 512, 128, 60, 60) == 1
     for T_q in (1, 8, 137, 512, 1024):
         for keys in (64, 700, 9000, 10 ** 6):
-            s = L.halo_prefill_splits(1, 32, 8, T_q, 128, keys, min(keys, T_q))
+            s = L.halo_prefill_splits(nat.BF16, 1, 32, 8, T_q, 128, keys, min(keys, T_q))
             assert 1 <= s <= min(32, -(-keys // 64))
-            assert (L.halo_prefill_workspace_size(1, 32, 8, T_q, 128, s) > 0) == (s > 1)
+            assert (L.halo_prefill_workspace_size(nat.BF16, 1, 32, 8, T_q, 128, s) > 0) == (s > 1)
