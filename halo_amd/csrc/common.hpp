@@ -105,6 +105,115 @@ __device__ __forceinline__ float load_elem(const void* base, int64_t idx, int dt
   return dtype == HALO_BF16 ? __uint_as_float((uint32_t)h << 16) : f16_bits_to_f32(h);
 }
 
+// The 16/esz elements of one 16-byte piece as fp32.
+template <int DT>
+__device__ __forceinline__ void unpack16(const uint4& v, float* f) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if constexpr (DT == HALO_F32) {
+      f[e] = __uint_as_float(w[e]);
+    } else if constexpr (DT == HALO_BF16) {
+      f[2 * e] = bf16_lo(w[e]);
+      f[2 * e + 1] = bf16_hi(w[e]);
+    } else {
+      f[2 * e] = f16_bits_to_f32((uint16_t)(w[e] & 0xffffu));
+      f[2 * e + 1] = f16_bits_to_f32((uint16_t)(w[e] >> 16));
+    }
+  }
+}
+
+// Store 16/esz consecutive fp32 values as elements `DT`: one 16-byte store
+// where `vec` says the destination is aligned for it, else element stores.
+template <int DT>
+__device__ __forceinline__ void store_piece(void* base, int64_t idx, bool vec, const float* v) {
+  constexpr int EPC = DT == HALO_F32 ? 4 : 8;
+  if (vec) {
+#pragma unroll
+    for (int e = 0; e < EPC; e += 4) store_elem4(base, idx + e, DT, v + e);
+  } else {
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) store_elem(base, idx + e, DT, v[e]);
+  }
+}
+
+// Slice c of the GQA-mean query of one KV head: elements ep*(c + pp*G) + e
+// (pp < 16/ep, e < ep, ep = elements of a 16-byte piece) of the mean of the
+// `rep` query heads from head h*rep on, added in head order, multiplied by
+// fp32(1/rep) and rounded to the query dtype (torch's .mean keeps it); rep
+// == 1 takes the head as it is.  `qb` is the element offset of head 0; `vec`:
+// every head row is 16-byte aligned.
+template <int DT>
+__device__ __forceinline__ void gqa_mean_slice(const void* q, int64_t qb, int64_t qsh, int h, int rep, float inv_rep,
+                                               int c, int G, bool vec, float (&out)[16]) {
+  constexpr int ep = DT == HALO_F32 ? 4 : 8;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) out[i] = 0.f;
+  // four heads at a time: their loads are independent and in flight together
+  for (int j0 = 0; j0 < rep; j0 += 4) {
+    float x[4][16];
+    if (vec) {
+      uint4 v[4][16 / ep];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t hb = qb + (int64_t)(h * rep + min(j0 + j, rep - 1)) * qsh;
+#pragma unroll
+        for (int pp = 0; pp < 16 / ep; ++pp)
+          v[j][pp] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(q) +
+                                                     (hb + (int64_t)ep * (c + pp * G)) * (16 / ep));
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int pp = 0; pp < 16 / ep; ++pp) unpack16<DT>(v[j][pp], x[j] + pp * ep);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t hb = qb + (int64_t)(h * rep + min(j0 + j, rep - 1)) * qsh;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[j][i] = load_elem(q, hb + (int64_t)ep * (c + (i / ep) * G) + i % ep, DT);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j0 + j < rep) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) out[i] = rep == 1 ? x[j][i] : out[i] + x[j][i];
+      }
+  }
+  if (rep != 1) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float a = opaque(out[i] * inv_rep);  // fp32 product, then one rounding to the q dtype
+      out[i] = DT == HALO_F32 ? a
+               : (DT == HALO_BF16 ? __uint_as_float((uint32_t)f32_to_bf16_rne(a) << 16)
+                                  : f16_bits_to_f32(f32_to_f16_rne(a)));
+    }
+  }
+}
+
+// Sum of the G slice sums held by lanes c < G of a group of G2 lanes (G2 the
+// power of two at or above G), as a balanced pairwise tree in slice order;
+// lane 0 of the group holds the result.
+template <int G2>
+__device__ __forceinline__ float slice_tree(float a, int c, int G) {
+#pragma unroll
+  for (int s = 1; s < G2; s <<= 1) {
+    const float o = __shfl_xor(a, s, kWave);
+    if ((c ^ s) < G) a = __fadd_rn(a, o);
+  }
+  return a;
+}
+
+// Larger float <=> larger key (not for NaN).
+__device__ __forceinline__ uint32_t float_key(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float key_float(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+
 // ---------------------------------------------------------------------------
 // Wave-level reductions (wave64).
 // ---------------------------------------------------------------------------
