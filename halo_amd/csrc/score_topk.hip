@@ -78,6 +78,72 @@ __global__ void __launch_bounds__(256) chunk_means_kernel(const void* k, int64_t
   }
 }
 
+// The same for pages of at most RG rows, one to a row group: one thread per
+// 16-byte column piece of a page adds all its rows in row-group order, so the
+// means are the other kernel's bit for bit.  Such a page gives the kernel above
+// one load a thread in front of a barrier and an LDS pass: 8.4 us for 8192 rows
+// of 8 heads x 128 bf16 in 16-row pages, 5.4 here.
+template <int DT>
+__global__ void __launch_bounds__(256) chunk_means_col_kernel(const void* k, int64_t ksb, int64_t ksh, int64_t kst,
+                                                              int H_kv, int D, int64_t row0, int page, int n_pages,
+                                                              int64_t total, void* km, int64_t msb, int64_t msh,
+                                                              int64_t msp, int vec) {
+  constexpr int ESZ = DT == HALO_F32 ? 4 : 2;
+  constexpr int EPC = 16 / ESZ;
+  constexpr int U = 8;  // rows in flight
+  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (gid >= total) return;
+  const int SL = D / EPC;
+  const int col = (int)(gid % SL);
+  const int pg = (int)(gid / SL);
+  const int j = pg % n_pages, bh = pg / n_pages;
+  const int h = bh % H_kv, b = bh / H_kv;
+  const char* base = reinterpret_cast<const char*>(k) +
+                     ((int64_t)b * ksb + (int64_t)h * ksh + (row0 + (int64_t)j * page) * kst) * ESZ + col * 16;
+  float sum[EPC];
+#pragma unroll
+  for (int e = 0; e < EPC; ++e) sum[e] = 0.f;
+  for (int t0 = 0; t0 < page; t0 += U) {
+    uint4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)  // a row past the page is loaded as its last one and not used
+      v[u] = *reinterpret_cast<const uint4*>(base + (int64_t)min(t0 + u, page - 1) * kst * ESZ);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float f[EPC];
+      unpack16<DT>(v[u], f);
+      // adding +0 leaves a sum that began at +0 as it is
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) sum[e] += t0 + u < page ? f[e] : 0.f;
+    }
+  }
+  const float inv = 1.0f / (float)page;
+  const int64_t o = (int64_t)b * msb + (int64_t)h * msh + (int64_t)j * msp + col * EPC;
+  if constexpr (DT == HALO_F16) {
+    // The other kernel's product and conversion are one v_fma_mixlo_f16, which
+    // rounds once; written out here so that both give the same bits.
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t r = 0;
+      asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "+v"(r) : "v"(sum[2 * e]), "v"(inv));
+      asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(sum[2 * e + 1]), "v"(inv));
+      w[e] = r;
+    }
+    uint16_t* dst = reinterpret_cast<uint16_t*>(km) + o;
+    if (vec) {
+      *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dst[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < EPC; ++e) sum[e] *= inv;
+    store_piece<DT>(km, o, vec != 0, sum);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Score + top-k.  One workgroup per selection.  Selection s covers batch row
 // s (per_row) or every row (per_row == 0, the reference's amax over batch).
@@ -115,6 +181,7 @@ struct ScoreParams {
   const halo_chunk_desc* slot_catalog;
   int n_slots;
   int32_t* res_out;
+  int qvec;  // q rows are 16-byte aligned (score_pages_kernel)
 };
 
 constexpr int kMaxElig = 1024;
@@ -127,16 +194,106 @@ __device__ __forceinline__ bool beats(float sa, int ea, float sb, int eb) {
   return sa > sb || (sa == sb && ea < eb);
 }
 
+// Wave-wide selection of the kk largest of n <= 64*NX scores (lower position
+// first among equals, zeros of both signs equal): s_sel[i] = number of selected
+// positions before i, or -1.  The kk-th largest key is built bit by bit from
+// ballot counts (taken as int: `ties` goes below 0 once the equals are taken).
+template <int NX>
+__device__ __forceinline__ void select_ascending(const float* s_score, int n, int kk, int lane, int* s_sel) {
+  uint32_t key[NX];
+#pragma unroll
+  for (int x = 0; x < NX; ++x) {
+    const int i = 64 * x + lane;
+    key[x] = i < n ? float_key(s_score[i] + 0.f) : 0u;  // 0 is below the key of every score
+  }
+  uint32_t thr = 0;
+  for (int bit = 31; bit >= 0; --bit) {
+    const uint32_t trial = thr | (1u << bit);
+    int cnt = 0;
+#pragma unroll
+    for (int x = 0; x < NX; ++x) cnt += (int)__popcll(__ballot(key[x] >= trial));
+    if (cnt >= kk) thr = trial;
+    if (cnt == kk) break;
+  }
+  int ties = kk, pos0 = 0;
+#pragma unroll
+  for (int x = 0; x < NX; ++x) ties -= (int)__popcll(__ballot(key[x] > thr));
+  const uint64_t below = (1ull << lane) - 1;
+#pragma unroll
+  for (int x = 0; x < NX; ++x) {
+    const uint64_t eq = __ballot(key[x] == thr);
+    const bool take = key[x] > thr || (key[x] == thr && (int)__popcll(eq & below) < ties);
+    const uint64_t m = __ballot(take);
+    if (64 * x + lane < n) s_sel[64 * x + lane] = take ? pos0 + (int)__popcll(m & below) : -1;
+    pos0 += (int)__popcll(m);
+    ties -= (int)__popcll(eq);
+  }
+}
+
+// Raw scores of many pages, spread over the GPU: score_out[sel, i] = max over
+// (row, head) of qg . kbar, in the slice order of score_topk_kernel.  G = D/16
+// lanes per page, lane c on slice c, so a wave reads whole rows of 64/G2 pages;
+// the four waves of a workgroup take the (row, head) pairs in turn and meet in
+// LDS.  A launch bound by latency: one round trip for q and the page means.  With
+// the selection below, 512 pages x 8 heads x 128 took 67.5 us in one workgroup,
+// 6.1 + 8.4 here.
+template <int DT, int G2>
+__global__ void __launch_bounds__(256) score_pages_kernel(ScoreParams P, int tiles) {
+  constexpr int PPW = 64 / G2;  // pages per wave
+  constexpr int esz = DT == HALO_F32 ? 4 : 2;
+  constexpr int ep = 16 / esz;
+  __shared__ float s_best[4][PPW];
+  const int sel = blockIdx.x / tiles, tile = blockIdx.x % tiles;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b0 = P.per_row ? sel : 0;
+  const int nrh = (P.per_row ? 1 : P.B) * P.H_kv;
+  const int n = P.n_elig_per_sel ? min(P.n_elig_per_sel[sel], P.n_elig) : P.n_elig;
+  const int G = P.D / 16;
+  const int c = lane % G2, pw = lane / G2;
+  const int i = tile * PPW + pw;
+  const int chunk = i < n ? P.elig[(int64_t)sel * P.elig_stride + i] : 0;
+  float best = -INFINITY;
+  for (int rh = w; rh < nrh; rh += 4) {
+    const int r = rh / P.H_kv, h = rh % P.H_kv;
+    float a = 0.f;
+    if (c < G && i < n) {
+      const char* row = reinterpret_cast<const char*>(P.km) +
+                        ((int64_t)(b0 + r) * P.msb + (int64_t)h * P.msh + (int64_t)chunk * P.msp) * esz;
+      uint4 v[16 / ep];
+#pragma unroll
+      for (int p = 0; p < 16 / ep; ++p) v[p] = *reinterpret_cast<const uint4*>(row + (c + p * G) * 16);
+      float qg[16];
+      gqa_mean_slice<DT>(P.q, (int64_t)(b0 + r) * P.qsb, P.qsh, h, P.rep, P.inv_rep, c, G, P.qvec != 0, qg);
+#pragma unroll
+      for (int p = 0; p < 16 / ep; ++p) {
+        float f[ep];
+        unpack16<DT>(v[p], f);
+#pragma unroll
+        for (int e = 0; e < ep; ++e) a = __fadd_rn(a, __fmul_rn(qg[p * ep + e], f[e]));
+      }
+    }
+    best = fmaxf(best, slice_tree<G2>(a, c, G));
+  }
+  if (c == 0) s_best[w][pw] = best;
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < PPW && tile * PPW + t < n)
+    P.score_out[(int64_t)sel * P.n_elig + tile * PPW + t] =
+        fmaxf(fmaxf(s_best[0][t], s_best[1][t]), fmaxf(s_best[2][t], s_best[3][t]));
+}
+
 // DC: the head dim when known at compile time (64, 128, 256: the dot-product
 // loops unroll and every load of a triple is issued before the first use),
-// 0 for any other multiple of 16 (runtime loops).
+// 0 for any other multiple of 16 (runtime loops), -1: score_out holds the raw
+// scores (score_pages_kernel) and only the combination and the top-k remain.
 template <int DT, int DC>
 __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
-  __shared__ float s_qg[kMaxQg];
+  constexpr bool kGiven = DC < 0;
+  __shared__ float s_qg[kGiven ? 1 : kMaxQg];
   __shared__ __align__(16) float s_score[kMaxElig];
   __shared__ __align__(16) int s_chunk[kMaxElig];
   __shared__ __align__(16) int s_sel[kMaxElig];
-  __shared__ float s_dot[kMaxDots];
+  __shared__ float s_dot[kGiven ? 1 : kMaxDots];
   const int sel = blockIdx.x;
   const int tid = threadIdx.x;
   const int nthr = blockDim.x;
@@ -146,6 +303,14 @@ __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
   const int kk = min(P.k, n);
   const int32_t* elig = P.elig + (int64_t)sel * P.elig_stride;
 
+  for (int i = tid; i < n; i += nthr) s_chunk[i] = elig[i];
+  if constexpr (kGiven) {
+    for (int i = tid; i < n; i += nthr) {
+      const float v = P.score_out[(int64_t)sel * P.n_elig + i];
+      s_score[i] = v != v ? -INFINITY : v;
+    }
+    __syncthreads();
+  } else {
   // GQA mean of the query heads of each KV head, rounded to the q dtype
   // (torch's .mean keeps the dtype); rep == 1 uses q as is.
   const int Dq = DC ? DC : P.D;
@@ -177,7 +342,6 @@ __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
     }
     s_qg[i] = v;
   }
-  for (int i = tid; i < n; i += nthr) s_chunk[i] = elig[i];
   __syncthreads();
 
   // score[i] = max over (row, h) of sum_d qg * kbar.  One thread per
@@ -258,41 +422,43 @@ __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
   }
   for (int i = tid; i < n; i += nthr) s_score[i] = (s_score[i] != s_score[i]) ? -INFINITY : s_score[i];
   __syncthreads();
+  }  // !kGiven
 
   if (P.normalize) {
-    __shared__ float s_red[512];
-    // min over eligible pages, then max of (attn - min)
-    float mn = INFINITY;
-    for (int i = tid; i < n; i += nthr) mn = fminf(mn, s_score[i]);
-    s_red[tid] = mn;
-    __syncthreads();
-    for (int w = nthr / 2; w > 0; w >>= 1) {
-      if (tid < w) s_red[tid] = fminf(s_red[tid], s_red[tid + w]);
-      __syncthreads();
+    // min and max over the eligible pages; x - min grows with x, so the
+    // largest (attn - min) is (max - min).  Recency over all P_total pages:
+    // exp(-(P-1-p)/refresh), / (sum + 1e-12), / (max + 1e-12).  The partial
+    // sums of the 512 threads are added as a halving tree (t and t + 256, then
+    // t + 128, ...), whose last six levels are a wave's shuffles.
+    __shared__ float s_mn[8], s_mx[8], s_red[512];
+    const int lane = tid & 63;
+    float mn = INFINITY, mx = -INFINITY;
+    for (int i = tid; i < n; i += nthr) {
+      mn = fminf(mn, s_score[i]);
+      mx = fmaxf(mx, s_score[i]);
     }
-    mn = s_red[0];
-    __syncthreads();
-    float mx = -INFINITY;
-    for (int i = tid; i < n; i += nthr) mx = fmaxf(mx, s_score[i] - mn);
-    s_red[tid] = mx;
-    __syncthreads();
-    for (int w = nthr / 2; w > 0; w >>= 1) {
-      if (tid < w) s_red[tid] = fmaxf(s_red[tid], s_red[tid + w]);
-      __syncthreads();
-    }
-    mx = s_red[0];
-    __syncthreads();
-    // recency over all P_total pages: exp(-(P-1-p)/refresh), / (sum + 1e-12), / (max + 1e-12)
+    mn = -wave_max(-mn);
+    mx = wave_max(mx);
     const float dec = (float)max(P.refresh, 1);
     float rs = 0.f;
     for (int j = tid; j < P.P_total; j += nthr) rs += expf(-((float)(P.P_total - 1) - (float)j) / dec);
     s_red[tid] = rs;
-    __syncthreads();
-    for (int w = nthr / 2; w > 0; w >>= 1) {
-      if (tid < w) s_red[tid] += s_red[tid + w];
-      __syncthreads();
+    if (lane == 0) {
+      s_mn[tid >> 6] = mn;
+      s_mx[tid >> 6] = mx;
     }
-    const float rsum = s_red[0] + 1e-12f;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      mn = fminf(mn, s_mn[w]);
+      mx = fmaxf(mx, s_mx[w]);
+    }
+    mx -= mn;
+    float t4[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) t4[x] = s_red[lane + 64 * x] + s_red[lane + 64 * x + 256];
+    const float rtot = wave_sum((t4[0] + t4[2]) + (t4[1] + t4[3]));
+    const float rsum = rtot + 1e-12f;
     // the largest recency term is the last page's exp(0) = 1
     const float rmax = 1.0f / rsum + 1e-12f;
     for (int i = tid; i < n; i += nthr) {
@@ -307,43 +473,60 @@ __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
     __syncthreads();
   }
 
-  // Rank by (score desc, chunk asc); selected = rank < kk.  Candidates are
-  // read four at a time (16-byte LDS reads, several in flight); entries past
-  // n are padding that never outranks (-inf, index past every chunk).
-  for (int i = n + tid; i < ((n + 15) & ~15); i += nthr) {
-    s_score[i] = -INFINITY;
-    s_chunk[i] = 0x7fffffff;
-    s_sel[i] = 0;
-  }
-  __syncthreads();
+  // Selected chunks in ascending order.  An ascending eligible list (a page
+  // range, as the scorers pass it) is selected by wave 0 in registers; any
+  // other order is ranked by comparing every pair (512 pages with their
+  // scoring: 11.8 us, 38 in any other order).
+  bool up = true;
+  for (int i = tid; i < n; i += nthr) up = up && (i == 0 || s_chunk[i - 1] < s_chunk[i]);
+  const bool asc = __syncthreads_and(up);
   const int n16 = (n + 15) & ~15;
-  for (int i = tid; i < n; i += nthr) {
-    const float si = s_score[i];
-    const int ei = s_chunk[i];
-    int rank = 0;
-    for (int j = 0; j < n16; j += 16) {
-      float4 sv[4];
-      int4 ev[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        sv[x] = *reinterpret_cast<const float4*>(&s_score[j + 4 * x]);
-        ev[x] = *reinterpret_cast<const int4*>(&s_chunk[j + 4 * x]);
-      }
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        rank += (beats(sv[x].x, ev[x].x, si, ei) ? 1 : 0) + (beats(sv[x].y, ev[x].y, si, ei) ? 1 : 0) +
-                (beats(sv[x].z, ev[x].z, si, ei) ? 1 : 0) + (beats(sv[x].w, ev[x].w, si, ei) ? 1 : 0);
+  if (asc) {
+    if (tid < 64) {
+      if (n <= 64) select_ascending<1>(s_score, n, kk, tid, s_sel);
+      else if (n <= 128) select_ascending<2>(s_score, n, kk, tid, s_sel);
+      else if (n <= 256) select_ascending<4>(s_score, n, kk, tid, s_sel);
+      else if (n <= 512) select_ascending<8>(s_score, n, kk, tid, s_sel);
+      else select_ascending<16>(s_score, n, kk, tid, s_sel);
     }
-    s_sel[i] = rank < kk;
+  } else {
+    // rank by (score desc, chunk asc); selected = rank < kk.  Candidates are
+    // read four at a time (16-byte LDS reads, several in flight); entries past
+    // n are padding that never outranks (-inf, index past every chunk).
+    for (int i = n + tid; i < n16; i += nthr) {
+      s_score[i] = -INFINITY;
+      s_chunk[i] = 0x7fffffff;
+      s_sel[i] = 0;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += nthr) {
+      const float si = s_score[i];
+      const int ei = s_chunk[i];
+      int rank = 0;
+      for (int j = 0; j < n16; j += 16) {
+        float4 sv[4];
+        int4 ev[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          sv[x] = *reinterpret_cast<const float4*>(&s_score[j + 4 * x]);
+          ev[x] = *reinterpret_cast<const int4*>(&s_chunk[j + 4 * x]);
+        }
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          rank += (beats(sv[x].x, ev[x].x, si, ei) ? 1 : 0) + (beats(sv[x].y, ev[x].y, si, ei) ? 1 : 0) +
+                  (beats(sv[x].z, ev[x].z, si, ei) ? 1 : 0) + (beats(sv[x].w, ev[x].w, si, ei) ? 1 : 0);
+      }
+      s_sel[i] = rank < kk;
+    }
   }
   __syncthreads();
-  // Output slot = number of selected chunks with a smaller index (ascending).
+  // Output slot = number of selected chunks with a smaller index.
   for (int i = tid; i < n; i += nthr) {
     if (P.score_out) P.score_out[(int64_t)sel * P.n_elig + i] = s_score[i];
-    if (!s_sel[i]) continue;
+    if (asc ? s_sel[i] < 0 : !s_sel[i]) continue;
     const int ei = s_chunk[i];
-    int pos = 0;
-    for (int j = 0; j < n16; j += 16) {
+    int pos = asc ? s_sel[i] : 0;
+    for (int j = asc ? n16 : 0; j < n16; j += 16) {
       int4 sv[4], ev[4];
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
@@ -412,10 +595,28 @@ extern "C" int halo_chunk_means(const void* k, int64_t k_stride_b, int64_t k_str
                  "key rows must be 16-byte aligned");
   const int64_t blocks = (int64_t)B * H_kv * n_pages;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int es = elem_size(dtype);
+  const int SL = D / (16 / es), RG = 256 / SL;
+  // Whole pages per thread for pages of up to 16 rows, and longer ones that give
+  // 64K threads, while a row group holds one row; 256 threads a page otherwise.
+  // bf16, here / 256 threads a page: 16-row pages of 8 heads x 128, 8192 rows 4.0 /
+  // 6.9 us, 32768 rows 15.0 / 20.4; 32-row pages of 8 heads x 64, 8192 rows (16K
+  // threads) 4.4 / 4.4, 32768 rows 5.4 / 10.7.
+  const int64_t total = blocks * SL;
+  const bool col = page <= RG && (page <= 16 || total >= 65536);
+  const int vec = reinterpret_cast<uintptr_t>(kmean) % 16 == 0 && (km_stride_b * es) % 16 == 0 &&
+                  (km_stride_h * es) % 16 == 0 && (km_stride_p * es) % 16 == 0;
 #define HALO_MEANS(DTV)                                                                                  \
-  hipLaunchKernelGGL(chunk_means_kernel<DTV>, dim3((unsigned)blocks), dim3(256), 0, st, k, k_stride_b,   \
-                     k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, kmean, km_stride_b, km_stride_h, \
-                     km_stride_p)
+  do {                                                                                                   \
+    if (col)                                                                                             \
+      hipLaunchKernelGGL(chunk_means_col_kernel<DTV>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, k, \
+                         k_stride_b, k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, total, kmean, \
+                         km_stride_b, km_stride_h, km_stride_p, vec);                                    \
+    else                                                                                                 \
+      hipLaunchKernelGGL(chunk_means_kernel<DTV>, dim3((unsigned)blocks), dim3(256), 0, st, k, k_stride_b, \
+                         k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, kmean, km_stride_b, km_stride_h, \
+                         km_stride_p);                                                                   \
+  } while (0)
   if (dtype == HALO_F32) HALO_MEANS(HALO_F32);
   else if (dtype == HALO_BF16) HALO_MEANS(HALO_BF16);
   else HALO_MEANS(HALO_F16);
@@ -494,7 +695,35 @@ static int score_topk_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h
   p.res_out = res_out;
   HALO_CHECK_ARG(!normalize || P_total > 0, "P_total must be positive when normalising");
   const int n_sel = per_row ? B : 1;
+  const int es = elem_size(dtype);
+  p.qvec = reinterpret_cast<uintptr_t>(q) % 16 == 0 && (q_stride_b * es) % 16 == 0 && (q_stride_h * es) % 16 == 0;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // Scores on their own grid, held by score_out until the selection reads
+  // them, where one CU would walk the means for longer than a launch costs.
+  // Own grid / one workgroup, at 8 heads x 128 bf16: 16 pages 8.3 / 8.4 us, 32
+  // 8.9 / 9.1, 64 8.8 / 10.8, 512 11.8 / 38; at 4 heads x 64: 64 pages 7.3 / 6.6,
+  // 128 7.6 / 7.8, 512 9.9 / 15.3.
+  if (score_out != nullptr && (int64_t)n_elig * nrows * H_kv * D >= 32768) {
+    const int G = D / 16;
+    const int G2 = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : G <= 8 ? 8 : 16;
+    const int tiles = (n_elig + 64 / G2 - 1) / (64 / G2);
+    const dim3 grid((unsigned)(n_sel * tiles));
+#define HALO_PAGES(DTV)                                                                                        \
+  do {                                                                                                         \
+    if (G2 == 1) hipLaunchKernelGGL((score_pages_kernel<DTV, 1>), grid, dim3(256), 0, st, p, tiles);           \
+    else if (G2 == 2) hipLaunchKernelGGL((score_pages_kernel<DTV, 2>), grid, dim3(256), 0, st, p, tiles);      \
+    else if (G2 == 4) hipLaunchKernelGGL((score_pages_kernel<DTV, 4>), grid, dim3(256), 0, st, p, tiles);      \
+    else if (G2 == 8) hipLaunchKernelGGL((score_pages_kernel<DTV, 8>), grid, dim3(256), 0, st, p, tiles);      \
+    else hipLaunchKernelGGL((score_pages_kernel<DTV, 16>), grid, dim3(256), 0, st, p, tiles);                  \
+    hipLaunchKernelGGL((score_topk_kernel<DTV, -1>), dim3(n_sel), dim3(512), 0, st, p);                        \
+  } while (0)
+    if (dtype == HALO_F32) HALO_PAGES(HALO_F32);
+    else if (dtype == HALO_BF16) HALO_PAGES(HALO_BF16);
+    else HALO_PAGES(HALO_F16);
+#undef HALO_PAGES
+    HALO_CHECK_HIP(hipGetLastError());
+    return HALO_OK;
+  }
 #define HALO_SCORE(DTV)                                                                                    \
   do {                                                                                                     \
     if (D == 64) hipLaunchKernelGGL((score_topk_kernel<DTV, 64>), dim3(n_sel), dim3(512), 0, st, p);       \
