@@ -111,81 +111,167 @@ struct KiviQuantParams {
   int vec16;         // K and V rows 16-byte aligned: tiles loaded with 16-byte loads
 };
 
-// Code of x for a group with precomputed inv = 1/scale (correctly rounded):
-// clamp(rint(dtype(dtype(x - zero) / scale)), 0, qmax).  The fp32 quotient
-// is formed without a division: q = d * inv, r = fma(-q, scale, d),
-// q' = fma(r, inv, q) equals the correctly rounded d / scale whenever d
-// (a dtype value >= 0) is 0 or in [2^-63, 2^63] and scale is in [2^-63,
-// 2^63] -- checked exhaustively for every pair of fp16 and bf16 values.
-// Outside that range (a zero scale, extreme bf16 values) the division runs.
-__device__ __forceinline__ float kivi_scale_ok(float scale) {
-  return scale >= 0x1p-63f && scale <= 0x1p63f ? 1.f : 0.f;
+// Keeps an fp32 value from being folded into the conversion behind it.
+__device__ __forceinline__ float pin(float x) {
+  asm("" : "+v"(x));
+  return x;
 }
-// p = (scale, 1/scale, zero, kivi_scale_ok(scale))
-template <int DT, int BITS>
-__device__ __forceinline__ uint32_t kivi_code_fma(float x, float4 p) {
-  constexpr float qmax = (float)((1 << BITS) - 1);
-  const float scale = p.x, inv = p.y, zero = p.z;
-  const float d = round_dt<DT>(opaque(x - zero));
-  const bool s_ok = p.w != 0.f;
-  const bool ok = DT == HALO_F16 ? s_ok : (s_ok && (d == 0.f || (d >= 0x1p-63f && d <= 0x1p63f)));
-  float q;
-  if (ok) {
-    const float q0 = opaque(d * inv);
-    const float r = __builtin_fmaf(-q0, scale, d);
-    q = __builtin_fmaf(r, inv, q0);
+
+// Two values rounded to the dtype; bf16 in one v_cvt_pk_bf16_f32.
+template <int DT>
+__device__ __forceinline__ void round_pair(float& a, float& b) {
+  if constexpr (DT == HALO_BF16) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+    const b2 v = {(__bf16)a, (__bf16)b};
+    const uint32_t w = __builtin_bit_cast(uint32_t, v);
+    a = bf16_lo(w);
+    b = bf16_hi(w);
   } else {
-    q = opaque(d / scale);
-  }
-  if constexpr (DT == HALO_F16) {
-    // ratio in fp16; NaN -> 0 through the IEEE max, codes in [0, qmax]
-    const _Float16 r16 = (_Float16)q;
-    _Float16 c16 = __builtin_rintf16(r16);
-    c16 = __builtin_fminf16(__builtin_fmaxf16(c16, (_Float16)0.f), (_Float16)qmax);
-    return (uint32_t)(unsigned short)c16;
-  } else {
-    const float ratio = round_dt<DT>(q);
-    return (uint32_t)fminf(fmaxf(rintf(ratio), 0.f), qmax);
+    a = (float)(_Float16)pin(a);
+    b = (float)(_Float16)pin(b);
   }
 }
 
-// Store a thread's NB packed code bytes (NB in {2, 4, 8, 16, 32}; dst aligned
-// to min(NB, 16) bytes) with vector stores.
-template <int NB>
-__device__ __forceinline__ void store_codes(uint8_t* dst, const uint64_t (&acc)[4]) {
-  static_assert(NB == 2 || NB == 4 || NB == 8 || NB == 16 || NB == 32, "packed code bytes per thread");
-  if constexpr (NB == 2) {
-    *reinterpret_cast<uint16_t*>(dst) = (uint16_t)acc[0];
-  } else if constexpr (NB == 4) {
-    *reinterpret_cast<uint32_t*>(dst) = (uint32_t)acc[0];
-  } else if constexpr (NB == 8) {
-    *reinterpret_cast<uint64_t*>(dst) = acc[0];
-  } else {
+// Codes of x without a division: with inv = 1/scale correctly rounded, d =
+// dtype(x - zero) >= 0, q = d * inv, r = fma(-q, scale, d), the quotient q' =
+// fma(r, inv, q) equals the correctly rounded d / scale whenever d is 0 or in
+// [2^-63, 2^63] and scale is in [2^-63, 2^63] -- checked exhaustively for every
+// pair of fp16 and bf16 values.  Scales of [2^-60, 2^50] are taken here, so that
+// d <= 2^8 * scale * (1 + 2^-7) stays in range above, and below 2^-63 both the
+// quotient and q' are under 1/4: code 0.  A zero scale (an fp16 group whose
+// range rounds to 0 in qmax parts) goes with inv = 2^100: d = 0 gives 0 (as the
+// NaN of 0 / 0 does) and any other d infinity in fp16, as d / 0 does.
+__device__ __forceinline__ bool kivi_scale_ok(float scale) {
+  return (scale >= 0x1p-60f && scale <= 0x1p50f) || scale == 0.f;
+}
+__device__ __forceinline__ float4 kivi_code_params(float scale, float zero) {
+  return make_float4(scale, scale == 0.f ? 0x1p100f : 1.0f / scale, zero, 0.f);
+}
+// codes of two elements, as floats; p = (scale, inv, zero, -) of each
+template <int DT, int BITS>
+__device__ __forceinline__ void kivi_code_pair(float& a, float& b, const float4& pa, const float4& pb) {
+  constexpr float qmax = (float)((1 << BITS) - 1);
+  a -= pa.z;
+  b -= pb.z;
+  round_pair<DT>(a, b);
+  const float qa = pin(a * pa.y), qb = pin(b * pb.y);
+  a = __builtin_fmaf(__builtin_fmaf(-qa, pa.x, a), pa.y, qa);
+  b = __builtin_fmaf(__builtin_fmaf(-qb, pb.x, b), pb.y, qb);
+  round_pair<DT>(a, b);
+  // clamp in one operation; of a NaN it is the smallest of the others, 0
+  a = __builtin_amdgcn_fmed3f(rintf(a), 0.f, qmax);
+  b = __builtin_amdgcn_fmed3f(rintf(b), 0.f, qmax);
+}
+// min(a, x, y) and max(a, x, y), NaN dropped, in one operation each
+__device__ __forceinline__ float kmin3(float a, float x, float y) {
+  float r;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(x), "v"(y));
+  return r;
+}
+__device__ __forceinline__ float kmax3(float a, float x, float y) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(x), "v"(y));
+  return r;
+}
+
+// Codes of one block from its staged tiles.  An 8-element run is 8 * BITS bits,
+// collected as BITS/2 fp32 sums of code * 2^position (16 bits each: exact).
+template <int DT, int D, int BITS, bool FAST>
+__device__ __forceinline__ void kivi_store_codes(const uint16_t* s_k, const uint16_t* s_v, const float4* s_kp,
+                                                 const float4* s_vp, uint8_t* out) {
+  constexpr int G = kKiviG, NG = D / G, RS = D + 8, C = kivi_code_bytes(D, BITS);
+  constexpr int NW = BITS / 2;  // 16-bit words of an 8-element run
+  const int tid = threadIdx.x;
+  auto codes = [](float& a, float& b, const float4& pa, const float4& pb) {
+    if constexpr (FAST) {
+      kivi_code_pair<DT, BITS>(a, b, pa, pb);
+    } else {
+      a = (float)kivi_code<DT, BITS>(a, pa.x, pa.z);
+      b = (float)kivi_code<DT, BITS>(b, pb.x, pb.z);
+    }
+  };
+  auto put_words = [](uint8_t* dst, const float (&sum)[NW]) {  // BITS bytes
+    if constexpr (BITS == 2) {
+      *reinterpret_cast<uint16_t*>(dst) = (uint16_t)(uint32_t)sum[0];
+    } else if constexpr (BITS == 4) {
+      *reinterpret_cast<uint32_t*>(dst) = (uint32_t)sum[0] | (uint32_t)sum[1] << 16;
+    } else {
+      *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)sum[0] | (uint32_t)sum[1] << 16,
+                                                  (uint32_t)sum[2] | (uint32_t)sum[3] << 16);
+    }
+  };
+  // K: 32 rows x D elements; thread = (8 channels, D/64 tokens), so that the
+  // parameters of its channels, the larger part of the LDS reads, are read once
+  {
+    constexpr int TT = D / 64;
+    const int oct = tid % (D / 8), t0 = (tid / (D / 8)) * TT;
+    float sum[TT][NW] = {};
+    uint4 r[TT];
 #pragma unroll
-    for (int h = 0; h < NB / 16; ++h)
-      reinterpret_cast<uint4*>(dst)[h] = make_uint4((uint32_t)acc[2 * h], (uint32_t)(acc[2 * h] >> 32),
-                                                    (uint32_t)acc[2 * h + 1], (uint32_t)(acc[2 * h + 1] >> 32));
+    for (int t = 0; t < TT; ++t) r[t] = *reinterpret_cast<const uint4*>(&s_k[(t0 + t) * RS + 8 * oct]);
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const float4 pa = s_kp[9 * oct + i], pb = s_kp[9 * oct + i + 1];
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const uint32_t w = i == 0 ? r[t].x : i == 2 ? r[t].y : i == 4 ? r[t].z : r[t].w;
+        float a = from_bits<DT>((uint16_t)w), c = from_bits<DT>((uint16_t)(w >> 16));
+        codes(a, c, pa, pb);
+        const int b0 = kivi_bit<BITS>(i), b1 = kivi_bit<BITS>(i + 1);
+        sum[t][b0 >> 4] = __builtin_fmaf(a, (float)(1 << (b0 & 15)), sum[t][b0 >> 4]);
+        sum[t][b1 >> 4] = __builtin_fmaf(c, (float)(1 << (b1 & 15)), sum[t][b1 >> 4]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TT; ++t) put_words(out + (t0 + t) * (D * BITS / 8) + oct * BITS, sum[t]);
+  }
+  // V: D rows (channels) x 32 slots; thread = (two channels, 8 consecutive slots)
+  constexpr int VRB = G * BITS / 8;          // V code bytes per channel row
+  for (int u = tid; u < 2 * D; u += 256) {
+    const int d = 2 * (u >> 2), o = u & 3;
+    const int g = d / G;
+    float sum[2][NW] = {};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int t = (i & 4 ? 16 : 0) + 4 * o + (i & 3);  // kivi_vtok(8 * o + i)
+      const float4 pv = s_vp[t * NG + g];
+      const uint32_t w = *reinterpret_cast<const uint32_t*>(&s_v[t * RS + d]);
+      float a = from_bits<DT>((uint16_t)w), c = from_bits<DT>((uint16_t)(w >> 16));
+      codes(a, c, pv, pv);
+      const int bit = kivi_bit<BITS>(i);
+      sum[0][bit >> 4] = __builtin_fmaf(a, (float)(1 << (bit & 15)), sum[0][bit >> 4]);
+      sum[1][bit >> 4] = __builtin_fmaf(c, (float)(1 << (bit & 15)), sum[1][bit >> 4]);
+    }
+    put_words(out + C + 4 * D + d * VRB + o * BITS, sum[0]);
+    put_words(out + C + 4 * D + (d + 1) * VRB + o * BITS, sum[1]);
   }
 }
 
 // One workgroup per block, 256 threads.  The 32 x D K and V tiles are staged
 // in LDS in their storage dtype (16-byte loads; rows padded by 16 bytes so
-// column and row-run reads spread over the banks); pairs of threads reduce
-// each K channel and each V (token, 32-channel group) to its min / max;
-// then each thread codes a run of consecutive elements of one output row
-// and stores its packed bytes in one store (K rows token-major, V rows
-// channel-major in slot order), so every global access is a vector access.
+// column and row-run reads spread over the banks); 512/D threads reduce each
+// pair of K channels and two each V (token, 32-channel group) to its min / max;
+// then each thread codes 8 channels of D/64 output rows (K, token-major) and
+// two channels x 8 slots (V, channel-major in slot order) and stores packed
+// bytes.  An element costs about 14 VALU operations (bf16 rounding in hardware
+// two at a time, no per-element range branch, codes packed by fp32
+// multiply-adds of up to 16 bits), where rounding by hand and a checked quotient
+// took 23 in fp16 and more than twice that in bf16.  32768 tokens x 8 heads x 128
+// bf16 in 2 bits: 102.9 us before, 46.2 now (3.4 TB/s), bound by the phases
+// behind its barriers.  Workgroups that walk several blocks with the next
+// block's loads in flight took 69: the barriers wait for those loads.
 template <int DT, int D, int BITS>
 __global__ void __launch_bounds__(256) kivi_quantize_kernel(KiviQuantParams P) {
   constexpr int G = kKiviG;
   constexpr int C = kivi_code_bytes(D, BITS);
   constexpr int NG = D / G;                  // V groups per token
   constexpr int RS = D + 8;                  // LDS row stride (elements)
-  constexpr int KR = G * D / 256;            // elements per thread per code run: 8, 16 or 32
-  constexpr int KP = D + D / KR;             // padded params (one float4 per channel, a pad per run)
+  constexpr int KP = D + D / 8;              // padded params (one float4 per channel, a pad per 8)
   __shared__ __align__(16) uint16_t s_k[G * RS], s_v[G * RS];
-  __shared__ float s_kmn[2][D], s_kmx[2][D], s_vmn[2][G * NG], s_vmx[2][G * NG];
-  __shared__ __align__(16) float4 s_kp[KP];  // (scale, 1/scale, zero, scale in range) per channel
+  constexpr int NP = 512 / D, PT = G / NP;   // partial K ranges per channel, of PT tokens: a pair per thread
+  __shared__ __align__(8) float s_kmn[NP][D], s_kmx[NP][D];
+  __shared__ float s_vmn[2][G * NG], s_vmx[2][G * NG];
+  __shared__ __align__(16) float4 s_kp[KP];  // kivi_code_params per channel
   __shared__ __align__(16) float4 s_vp[G * NG];
   const int tid = threadIdx.x;
   const int j = blockIdx.x % P.n_blk;
@@ -218,18 +304,28 @@ __global__ void __launch_bounds__(256) kivi_quantize_kernel(KiviQuantParams P) {
     }
   }
   __syncthreads();
-  // min / max: K per (channel, half of the tokens), V per (token, group, half of the channels)
-  for (int i = tid; i < 2 * D; i += 256) {
-    const int d = i % D, hf = i / D;
-    float mn = from_bits<DT>(s_k[(16 * hf) * RS + d]), mx = mn;
+  // min / max: K per (two channels, PT of the tokens), V per (token, group, half of the channels)
+  {
+    const int d = 2 * (tid % (D / 2)), qt = tid / (D / 2);
+    uint32_t w[PT];
 #pragma unroll
-    for (int t = 1; t < 16; ++t) {
-      const float x = from_bits<DT>(s_k[(16 * hf + t) * RS + d]);
-      mn = fminf(mn, x);
-      mx = fmaxf(mx, x);
+    for (int t = 0; t < PT; ++t) w[t] = *reinterpret_cast<const uint32_t*>(&s_k[(PT * qt + t) * RS + d]);
+    float mn[2], mx[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float x[PT];
+#pragma unroll
+      for (int t = 0; t < PT; ++t) x[t] = from_bits<DT>((uint16_t)(c ? w[t] >> 16 : w[t]));
+      mn[c] = fminf(x[0], x[1]);
+      mx[c] = fmaxf(x[0], x[1]);
+#pragma unroll
+      for (int t = 2; t < PT; t += 2) {
+        mn[c] = kmin3(mn[c], x[t], x[t + 1]);
+        mx[c] = kmax3(mx[c], x[t], x[t + 1]);
+      }
     }
-    s_kmn[hf][d] = mn;
-    s_kmx[hf][d] = mx;
+    *reinterpret_cast<float2*>(&s_kmn[qt][d]) = make_float2(mn[0], mn[1]);
+    *reinterpret_cast<float2*>(&s_kmx[qt][d]) = make_float2(mx[0], mx[1]);
   }
   for (int i = tid; i < 2 * G * NG; i += 256) {
     const int tg = i >> 1, hf = i & 1;
@@ -241,8 +337,8 @@ __global__ void __launch_bounds__(256) kivi_quantize_kernel(KiviQuantParams P) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       const float lo = from_bits<DT>((uint16_t)w[c]), hi = from_bits<DT>((uint16_t)(w[c] >> 16));
-      mn = fminf(mn, fminf(lo, hi));
-      mx = fmaxf(mx, fmaxf(lo, hi));
+      mn = kmin3(mn, lo, hi);
+      mx = kmax3(mx, lo, hi);
     }
     s_vmn[hf][tg] = mn;
     s_vmx[hf][tg] = mx;
@@ -251,65 +347,33 @@ __global__ void __launch_bounds__(256) kivi_quantize_kernel(KiviQuantParams P) {
   uint8_t* out = P.blocks + (int64_t)b * P.bsb + (int64_t)h * P.bsh + (int64_t)j * kivi_block_bytes(D, BITS);
   uint16_t* meta_k = reinterpret_cast<uint16_t*>(out + C);
   uint16_t* meta_v = reinterpret_cast<uint16_t*>(out + 2 * C + 4 * D);
+  bool ok = true;
   for (int d = tid; d < D; d += 256) {
     float sc, z;
-    kivi_params<DT, BITS>(fminf(s_kmn[0][d], s_kmn[1][d]), fmaxf(s_kmx[0][d], s_kmx[1][d]), sc, z);
-    s_kp[d + d / KR] = make_float4(sc, 1.0f / sc, z, kivi_scale_ok(sc));
+    float mn = s_kmn[0][d], mx = s_kmx[0][d];
+#pragma unroll
+    for (int p = 1; p < NP; ++p) {
+      mn = fminf(mn, s_kmn[p][d]);
+      mx = fmaxf(mx, s_kmx[p][d]);
+    }
+    kivi_params<DT, BITS>(mn, mx, sc, z);
+    s_kp[d + d / 8] = kivi_code_params(sc, z);
+    ok = ok && kivi_scale_ok(sc);
     meta_k[d] = bits_dt<DT>(sc);
     meta_k[D + d] = bits_dt<DT>(z);
   }
   for (int tg = tid; tg < G * NG; tg += 256) {
     float sc, z;
     kivi_params<DT, BITS>(fminf(s_vmn[0][tg], s_vmn[1][tg]), fmaxf(s_vmx[0][tg], s_vmx[1][tg]), sc, z);
-    s_vp[tg] = make_float4(sc, 1.0f / sc, z, kivi_scale_ok(sc));
+    s_vp[tg] = kivi_code_params(sc, z);
+    ok = ok && kivi_scale_ok(sc);
     const int t = tg / NG, g = tg % NG;
     meta_v[g * G + kivi_vslot(t)] = bits_dt<DT>(sc);            // group-major, slot order
     meta_v[G * NG + g * G + kivi_vslot(t)] = bits_dt<DT>(z);
   }
-  __syncthreads();
-  // K codes: 32 rows x D elements; thread = (token, run of KR consecutive
-  // channels starting at a multiple of 8), KR * BITS bits stored at once
-  constexpr int RKB = D * BITS / 8;          // K code bytes per token row
-  {
-    const int t = tid / (D / KR), e0 = (tid % (D / KR)) * KR;
-    uint64_t acc[4] = {0, 0, 0, 0};          // up to 256 bits (32 elements x 8 bits)
-    const uint4* row = reinterpret_cast<const uint4*>(&s_k[t * RS + e0]);
-#pragma unroll
-    for (int v8 = 0; v8 < KR / 8; ++v8) {
-      const uint4 r = row[v8];
-      const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int e = e0 + 8 * v8 + i;
-        const float4 pk = s_kp[e + e / KR];
-        const uint16_t xb = (uint16_t)(i & 1 ? w[i >> 1] >> 16 : w[i >> 1]);
-        const uint32_t c = kivi_code_fma<DT, BITS>(from_bits<DT>(xb), pk);
-        const int bit = kivi_bit<BITS>(8 * v8 + i);          // e0 is a multiple of 8
-        acc[bit >> 6] |= (uint64_t)c << (bit & 63);
-      }
-    }
-    uint8_t* dst = out + t * RKB + kivi_bit<BITS>(e0) / 8;
-    store_codes<KR * BITS / 8>(dst, acc);
-  }
-  // V codes: D rows (channels) x 32 slots; thread = (channel, run of VR
-  // consecutive slots starting at a multiple of 8)
-  constexpr int VR = G * D / 256;
-  constexpr int VRB = G * BITS / 8;          // V code bytes per channel row
-  {
-    const int d = tid / (G / VR), s0 = (tid % (G / VR)) * VR;
-    const int g = d / G;
-    uint64_t acc[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < VR; ++i) {
-      const int s = s0 + i, t = kivi_vtok(s);
-      const float4 pv = s_vp[t * NG + g];
-      const uint32_t c = kivi_code_fma<DT, BITS>(from_bits<DT>(s_v[t * RS + d]), pv);
-      const int bit = kivi_bit<BITS>(s) - kivi_bit<BITS>(s0);
-      acc[bit >> 6] |= (uint64_t)c << (bit & 63);
-    }
-    uint8_t* dst = out + C + 4 * D + d * VRB + kivi_bit<BITS>(s0) / 8;
-    store_codes<VR * BITS / 8>(dst, acc);
-  }
+  // every group's scale in range: no division; else all of the block divides
+  if (__syncthreads_and(ok)) kivi_store_codes<DT, D, BITS, true>(s_k, s_v, s_kp, s_vp, out);
+  else kivi_store_codes<DT, D, BITS, false>(s_k, s_v, s_kp, s_vp, out);
 }
 
 struct KiviDequantParams {
@@ -322,7 +386,90 @@ struct KiviDequantParams {
   int64_t vsb, vsh, vst;
 };
 
-// One workgroup per block; one thread per (token, 8-channel piece) of K and V.
+// One thread per (block, K or V, 8-channel piece c, lane group o): it turns the
+// codes of 8 channels x 8 tokens (K: tokens o + 4i; V: slots 8o..8o+7, whose
+// codes are one BITS-byte word a channel) with the scales and zeros of its piece
+// held in registers, and stores 16 bytes a token, so that a wave stores whole
+// rows.  K and V take the two halves of a workgroup.  32768 tokens x 8 heads x
+// 128 bf16 in 2 bits: 51.2 us with a thread per element (byte and 2-byte loads,
+// 2-byte stores), 28.2 here (5.7 TB/s).
+template <int DT, int D, int BITS>
+__global__ void __launch_bounds__(256) kivi_dequant_piece_kernel(KiviDequantParams P, int n) {
+  constexpr int G = kKiviG;
+  constexpr int C = kivi_code_bytes(D, BITS);
+  constexpr int NG = D / G;
+  constexpr int PR = D / 8;               // pieces per row
+  constexpr int NB = 128 / (4 * PR);      // blocks per workgroup
+  constexpr uint32_t MASK = (1u << BITS) - 1;
+  const bool is_v = threadIdx.x >= 128;
+  const int x = threadIdx.x & 127;
+  const int c = x % PR, o = (x / PR) & 3;
+  const int blk = blockIdx.x * NB + x / (4 * PR);
+  if (blk >= n) return;
+  const int j = blk % P.n_blk;
+  const int bh = blk / P.n_blk;
+  const int h = bh % P.H_kv, b = bh / P.H_kv;
+  const uint8_t* src = P.blocks + (int64_t)b * P.bsb + (int64_t)h * P.bsh + (int64_t)j * kivi_block_bytes(D, BITS);
+  // the 8 codes of word i: two 32-bit halves for 8-bit codes, one below
+  uint32_t code[8][BITS == 8 ? 2 : 1];
+  const uint8_t* cb = src + (is_v ? C + 4 * D + 8 * c * (G * BITS / 8) + o * BITS : o * (D * BITS / 8) + c * BITS);
+  const int step = is_v ? G * BITS / 8 : 4 * (D * BITS / 8);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (BITS == 2) {
+      code[i][0] = *reinterpret_cast<const uint16_t*>(cb + i * step);
+    } else if constexpr (BITS == 4) {
+      code[i][0] = *reinterpret_cast<const uint32_t*>(cb + i * step);
+    } else {
+      const uint2 w = *reinterpret_cast<const uint2*>(cb + i * step);
+      code[i][0] = w.x;
+      code[i][1] = w.y;
+    }
+  }
+  const uint8_t* meta = src + (is_v ? 2 * C + 4 * D + (c / 4) * 2 * G + 16 * o : C + 16 * c);
+  float sc[8], z[8];  // K: of the channels, V: of the slots
+  unpack16<DT>(*reinterpret_cast<const uint4*>(meta), sc);
+  unpack16<DT>(*reinterpret_cast<const uint4*>(meta + (is_v ? 2 * G * NG : 2 * D)), z);
+  auto at = [&](int w, int e) {  // code e of word w
+    const int bit = kivi_bit<BITS>(e);
+    return (float)((code[w][BITS == 8 ? bit >> 5 : 0] >> (bit & 31)) & MASK);
+  };
+  auto put = [&](uint16_t* base, int64_t row, const float* f) {
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (DT == HALO_BF16) {
+        typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+        const b2 v = {(__bf16)f[2 * e], (__bf16)f[2 * e + 1]};
+        w[e] = __builtin_bit_cast(uint32_t, v);
+      } else {
+        w[e] = (uint32_t)f32_to_f16_rne(pin(f[2 * e])) | (uint32_t)f32_to_f16_rne(pin(f[2 * e + 1])) << 16;
+      }
+    }
+    *reinterpret_cast<uint4*>(base + row + 8 * c) = make_uint4(w[0], w[1], w[2], w[3]);
+  };
+  if (!is_v) {
+    uint16_t* ko = reinterpret_cast<uint16_t*>(P.k) + (int64_t)b * P.ksb + (int64_t)h * P.ksh + (int64_t)j * G * P.kst;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = pin(at(i, e) * sc[e]) + z[e];
+      put(ko, (int64_t)(o + 4 * i) * P.kst, f);
+    }
+  } else {
+    uint16_t* vo = reinterpret_cast<uint16_t*>(P.v) + (int64_t)b * P.vsb + (int64_t)h * P.vsh + (int64_t)j * G * P.vst;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = pin(at(e, i) * sc[i]) + z[i];
+      put(vo, (int64_t)((i & 4 ? 16 : 0) + 4 * o + (i & 3)) * P.vst, f);
+    }
+  }
+}
+
+// Any alignment of blocks and rows: one thread per element.
 template <int DT, int D, int BITS>
 __global__ void __launch_bounds__(256) kivi_dequant_kernel(KiviDequantParams P) {
   constexpr int G = kKiviG;
@@ -373,13 +520,27 @@ int quant_bits(const KiviQuantParams& p, int bits, int n, hipStream_t st) {
   HALO_CHECK_HIP(hipGetLastError());
   return HALO_OK;
 }
-template <int DT, int D>
-int dequant_bits(const KiviDequantParams& p, int bits, int n, hipStream_t st) {
-  if (bits == 2) hipLaunchKernelGGL((kivi_dequant_kernel<DT, D, 2>), dim3(n), dim3(256), 0, st, p);
-  else if (bits == 4) hipLaunchKernelGGL((kivi_dequant_kernel<DT, D, 4>), dim3(n), dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((kivi_dequant_kernel<DT, D, 8>), dim3(n), dim3(256), 0, st, p);
+template <int DT, int D, int BITS>
+int dequant_run(const KiviDequantParams& p, int n, hipStream_t st) {
+  auto a16 = [](const void* q, int64_t sb, int64_t sh, int64_t s) {
+    return (reinterpret_cast<uintptr_t>(q) & 15) == 0 && sb % 16 == 0 && sh % 16 == 0 && s % 16 == 0;
+  };
+  // 16-byte loads and stores where blocks and rows allow them
+  if (a16(p.blocks, p.bsb, p.bsh, 0) && a16(p.k, 2 * p.ksb, 2 * p.ksh, 2 * p.kst) &&
+      a16(p.v, 2 * p.vsb, 2 * p.vsh, 2 * p.vst)) {
+    constexpr int NB = 256 / D;
+    hipLaunchKernelGGL((kivi_dequant_piece_kernel<DT, D, BITS>), dim3((n + NB - 1) / NB), dim3(256), 0, st, p, n);
+  } else {
+    hipLaunchKernelGGL((kivi_dequant_kernel<DT, D, BITS>), dim3(n), dim3(256), 0, st, p);
+  }
   HALO_CHECK_HIP(hipGetLastError());
   return HALO_OK;
+}
+template <int DT, int D>
+int dequant_bits(const KiviDequantParams& p, int bits, int n, hipStream_t st) {
+  if (bits == 2) return dequant_run<DT, D, 2>(p, n, st);
+  if (bits == 4) return dequant_run<DT, D, 4>(p, n, st);
+  return dequant_run<DT, D, 8>(p, n, st);
 }
 
 }  // namespace

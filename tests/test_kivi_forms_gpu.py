@@ -1,0 +1,58 @@
+"""The KIVI kernels at the edges of their forms: group scales on both sides of
+the range whose codes need no division (a block with one outside divides
+throughout), fp16 ranges that round to a zero scale, block counts off the
+dequantiser's blocks per workgroup, and buffers without 16-byte alignment.
+Blocks and values are the oracle's bit for bit."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import kivi as K
+from oracle.inputs import round_to
+
+pytestmark = pytest.mark.gpu
+TDT = {"bfloat16": torch.bfloat16, "float16": torch.float16}
+
+
+def _inputs(dtype, D, n):
+    rng = np.random.default_rng(D + n)
+    x = rng.standard_normal((2, 1, 1, 32 * n, D)).astype(np.float32)
+    if dtype == "bfloat16":  # per-token magnitudes: V groups far apart, K groups of the widest
+        x[:, :, :, 32:64] *= np.exp2(rng.integers(-100, -50, (32, 1))).astype(np.float32)
+        x[:, :, :, 64:96] *= np.exp2(rng.integers(45, 70, (32, 1))).astype(np.float32)
+    else:  # ranges of a few subnormal steps: the scale of range 1/qmax rounds to 0
+        x[:, :, :, 32:64] = rng.integers(-1, 2, (2, 1, 1, 32, D)) * 2.0 ** -24
+        x[:, :, :, 64:96, ::2] = 0.0
+    x[:, :, :, 96:128, :32] = np.where(rng.random((2, 1, 1, 32, 32)) < 0.5, 0.0, -0.0)
+    k, v = round_to(x[0], dtype), round_to(x[1], dtype)
+    return k, v
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("D,n", [(64, 5), (128, 5), (256, 4)])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_quantise_and_dequantise_forms(dev, dtype, D, n, bits):
+    from halo_amd import kivi
+    k, v = _inputs(dtype, D, n)
+    kt, vt = (torch.from_numpy(a).to(dev).to(TDT[dtype]) for a in (k, v))
+    blocks = kivi.quantize(kt, vt, bits=bits)
+    want = K.pack_blocks(k, v, bits=bits, dtype=dtype)
+    got = blocks.cpu().numpy()
+    # the sign of a zero minimum is not pinned: compare blocks without the signed zeros' run, all others whole
+    assert np.array_equal(np.delete(got, 3, axis=2), np.delete(want, 3, axis=2))
+    rk, rv = K.unpack_blocks(got, D=D, bits=bits, dtype=dtype)
+    kd, vd = kivi.dequantize(blocks, D=D, dtype=TDT[dtype], bits=bits)
+    assert np.array_equal(kd.float().cpu().numpy(), rk)
+    assert np.array_equal(vd.float().cpu().numpy(), rv)
+    # one byte row off 16: the element form
+    off = torch.empty(blocks.numel() + 8, device=dev, dtype=torch.uint8)[8:].view(blocks.shape)
+    off.copy_(blocks)
+    ku, vu = kivi.dequantize(off, D=D, dtype=TDT[dtype], bits=bits)
+    assert torch.equal(ku.view(torch.int16), kd.view(torch.int16))
+    assert torch.equal(vu.view(torch.int16), vd.view(torch.int16))
+    # rows off 16 bytes: the tiles are loaded by element
+    ke = torch.empty(kt.numel() + 1, device=dev, dtype=kt.dtype)[1:].view(kt.shape)
+    ke.copy_(kt)
+    assert torch.equal(kivi.quantize(ke, vt, bits=bits), blocks)
