@@ -16,6 +16,7 @@ from __future__ import annotations
 import collections
 import ctypes
 import math
+import struct
 from dataclasses import dataclass, field
 from typing import Optional, Sequence
 
@@ -32,7 +33,8 @@ DESC_DTYPE = np.dtype([
     ("vsb", "<i8"), ("vsh", "<i8"), ("vst", "<i8"),
     ("start", "<i8"), ("T", "<i4"), ("flags", "<i4"), ("batch", "<i4"), ("res", "<i4"),
 ])
-assert DESC_DTYPE.itemsize == 88
+_DESC = struct.Struct("<2Q7q4i")  # one record of DESC_DTYPE
+assert DESC_DTYPE.itemsize == _DESC.size == 88
 
 _WAVES_PER_GROUP = 4
 _TILE_ROWS = 64
@@ -105,14 +107,6 @@ def choose_rep_t(rep: int) -> int:
     return 8
 
 
-def _check_kv(t: torch.Tensor, name: str) -> None:
-    if t.stride(-1) != 1:
-        raise AssertionError(f"{name}: head dim must be contiguous (stride {t.stride()})")
-    esz = t.element_size()
-    if t.data_ptr() % 16 or (t.stride(-2) * esz) % 16:
-        raise AssertionError(f"{name}: rows must be 16-byte aligned")
-
-
 def _kernel_address(t: torch.Tensor, name: str) -> int:
     """Address a kernel reads ``t`` at: device memory as is; a chunk kept in
     pinned host memory (the cold tier) through its device-visible mapping,
@@ -169,6 +163,8 @@ def pack_descs(chunks: Sequence[ChunkRef], *, B: int, H_kv: int, D: int, dtype: 
     """halo_chunk_desc records for ``chunks`` (validated); returns
     (numpy structured array, list of tensors to keep alive)."""
     descs = np.zeros(len(chunks), dtype=DESC_DTYPE)
+    raw = descs.view(np.uint8).data  # a record is packed in one call: thirteen field stores cost 2 us a chunk
+    esz = dtype.itemsize
     keep = []
     for i, c in enumerate(chunks):
         if hasattr(c, "blocks"):
@@ -183,33 +179,32 @@ def pack_descs(chunks: Sequence[ChunkRef], *, B: int, H_kv: int, D: int, dtype: 
         k, v = c.k, c.v
         if k.dtype != dtype or v.dtype != dtype:
             raise AssertionError(f"chunk {i}: dtype {k.dtype}/{v.dtype} != {dtype}")
-        if k.shape[-1] != D or v.shape[-1] != D:
-            raise AssertionError(f"chunk {i}: head dim {k.shape[-1]}/{v.shape[-1]} != {D}")
-        if c.batch < 0:
-            if k.dim() != 4 or k.shape[0] != B or k.shape[1] != H_kv:
-                raise AssertionError(f"k shape {tuple(k.shape)} != ({B}, {H_kv}, T_c, {D})")
-            if tuple(v.shape) != tuple(k.shape):
-                raise AssertionError(f"v shape {tuple(v.shape)} != k shape {tuple(k.shape)}")
+        kn, vn, batch = k.shape, v.shape, c.batch
+        if kn[-1] != D or vn[-1] != D:
+            raise AssertionError(f"chunk {i}: head dim {kn[-1]}/{vn[-1]} != {D}")
+        ks, vs = k.stride(), v.stride()
+        if batch < 0:
+            if len(kn) != 4 or kn[0] != B or kn[1] != H_kv:
+                raise AssertionError(f"k shape {tuple(kn)} != ({B}, {H_kv}, T_c, {D})")
+            if vn != kn:
+                raise AssertionError(f"v shape {tuple(vn)} != k shape {tuple(kn)}")
+            strides = ks[:3] + vs[:3]
         else:
-            if k.dim() != 3 or k.shape[0] != H_kv or tuple(v.shape) != tuple(k.shape):
-                raise AssertionError(f"ragged chunk {i}: expected (H_kv, T_c, D), got {tuple(k.shape)}")
-            if not 0 <= c.batch < B:
-                raise AssertionError(f"ragged chunk {i}: batch {c.batch} outside [0, {B})")
-        _check_kv(k, f"chunk {i} k")
-        _check_kv(v, f"chunk {i} v")
+            if len(kn) != 3 or kn[0] != H_kv or vn != kn:
+                raise AssertionError(f"ragged chunk {i}: expected (H_kv, T_c, D), got {tuple(kn)}")
+            if not 0 <= batch < B:
+                raise AssertionError(f"ragged chunk {i}: batch {batch} outside [0, {B})")
+            strides = (0, ks[0], ks[1], 0, vs[0], vs[1])
+        kp, vp = k.data_ptr(), v.data_ptr()
+        for p, st, name in ((kp, ks, "k"), (vp, vs, "v")):
+            if st[-1] != 1:
+                raise AssertionError(f"chunk {i} {name}: head dim must be contiguous (stride {st})")
+            if p % 16 or (st[-2] * esz) % 16:
+                raise AssertionError(f"chunk {i} {name}: rows must be 16-byte aligned")
         keep += [k, v]
-        d = descs[i]
-        d["k"], d["v"] = _kernel_address(k, f"chunk {i} k"), _kernel_address(v, f"chunk {i} v")
-        if c.batch < 0:
-            d["ksb"], d["ksh"], d["kst"] = k.stride(0), k.stride(1), k.stride(2)
-            d["vsb"], d["vsh"], d["vst"] = v.stride(0), v.stride(1), v.stride(2)
-        else:
-            d["ksb"], d["ksh"], d["kst"] = 0, k.stride(0), k.stride(1)
-            d["vsb"], d["vsh"], d["vst"] = 0, v.stride(0), v.stride(1)
-        d["start"] = int(c.chunk_start)
-        d["T"] = c.T
-        d["flags"] = nat.CHUNK_CAUSAL if c.causal else 0
-        d["batch"] = int(c.batch)
+        _DESC.pack_into(raw, 88 * i, kp if k.is_cuda else _kernel_address(k, f"chunk {i} k"),
+                        vp if v.is_cuda else _kernel_address(v, f"chunk {i} v"), *strides, int(c.chunk_start), c.T,
+                        nat.CHUNK_CAUSAL if c.causal else 0, int(batch), 0)
     return descs, keep
 
 
