@@ -22,7 +22,12 @@ namespace halo {
 // whole coalesced rows and independent; the RG fp32 partial sums are then
 // added in row-group order through LDS and rounded once to the key dtype.
 // ---------------------------------------------------------------------------
-template <int DT>
+// U rows of a thread are in flight at a time: 8, 32 for 16-bit pages of at least 32
+// rows a thread, whose few workgroups are each bound by their own round trips
+// (one page of 1024 rows x 8 heads x 128 bf16, eight workgroups: 12.3 -> 5.7 us;
+// 256 rows 4.8 -> 3.0), or 0: left to the compiler (fp32, whose 1024 rows took 6.5
+// us so and 6.9-7.5 in batches).
+template <int DT, int U>
 __global__ void __launch_bounds__(256) chunk_means_kernel(const void* k, int64_t ksb, int64_t ksh, int64_t kst,
                                                           int H_kv, int D, int64_t row0, int page, int n_pages,
                                                           void* km, int64_t msb, int64_t msh, int64_t msp) {
@@ -42,27 +47,30 @@ __global__ void __launch_bounds__(256) chunk_means_kernel(const void* k, int64_t
   if (rg < RG) {
     const char* base = reinterpret_cast<const char*>(k) +
                        ((int64_t)b * ksb + (int64_t)h * ksh + (row0 + (int64_t)j * page) * kst) * ESZ + col * 16;
+    auto add = [&](const uint4& v) {
+      float x[EPC];
+      unpack16<DT>(v, x);
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) acc[e] += x[e];
+    };
+    int t = rg;
+    for (; U > 0 && t + (U - 1) * RG < page; t += U * RG) {
+      uint4 v[U > 0 ? U : 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const uint4*>(base + (int64_t)(t + u * RG) * kst * ESZ);
+#pragma unroll
+      for (int u = 0; u < U; ++u) add(v[u]);
+    }
+    if constexpr (U > 0) {
 #pragma unroll 8
-    for (int t = rg; t < page; t += RG) {
-      const uint4 v = *reinterpret_cast<const uint4*>(base + (int64_t)t * kst * ESZ);
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      if constexpr (DT == HALO_F32) {
+      for (; t < page; t += RG) add(*reinterpret_cast<const uint4*>(base + (int64_t)t * kst * ESZ));
+    } else {
+#pragma unroll 8
+      for (int r = rg; r < page; r += RG) {
+        const uint4 v = *reinterpret_cast<const uint4*>(base + (int64_t)r * kst * ESZ);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] += __uint_as_float(w[e]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float lo, hi;
-          if constexpr (DT == HALO_BF16) {
-            lo = bf16_lo(w[e]);
-            hi = bf16_hi(w[e]);
-          } else {
-            lo = f16_bits_to_f32((uint16_t)(w[e] & 0xffffu));
-            hi = f16_bits_to_f32((uint16_t)(w[e] >> 16));
-          }
-          acc[2 * e] += lo;
-          acc[2 * e + 1] += hi;
-        }
       }
     }
   }
@@ -612,10 +620,14 @@ extern "C" int halo_chunk_means(const void* k, int64_t k_stride_b, int64_t k_str
       hipLaunchKernelGGL(chunk_means_col_kernel<DTV>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, k, \
                          k_stride_b, k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, total, kmean, \
                          km_stride_b, km_stride_h, km_stride_p, vec);                                    \
+    else if (DTV != HALO_F32 && page >= 32 * RG)                                                         \
+      hipLaunchKernelGGL((chunk_means_kernel<DTV, DTV == HALO_F32 ? 0 : 32>), dim3((unsigned)blocks), dim3(256), 0, \
+                         st, k, k_stride_b, k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, kmean, \
+                         km_stride_b, km_stride_h, km_stride_p);                                         \
     else                                                                                                 \
-      hipLaunchKernelGGL(chunk_means_kernel<DTV>, dim3((unsigned)blocks), dim3(256), 0, st, k, k_stride_b, \
-                         k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, kmean, km_stride_b, km_stride_h, \
-                         km_stride_p);                                                                   \
+      hipLaunchKernelGGL((chunk_means_kernel<DTV, DTV == HALO_F32 ? 0 : 8>), dim3((unsigned)blocks), dim3(256), 0, \
+                         st, k, k_stride_b, k_stride_h, k_stride_t, H_kv, D, row0, page, n_pages, kmean, \
+                         km_stride_b, km_stride_h, km_stride_p);                                         \
   } while (0)
   if (dtype == HALO_F32) HALO_MEANS(HALO_F32);
   else if (dtype == HALO_BF16) HALO_MEANS(HALO_BF16);

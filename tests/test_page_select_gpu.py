@@ -38,6 +38,8 @@ def _off(x):
     (torch.float16, 128, 11, 50),
     (torch.float32, 128, 8, 41), (torch.float32, 128, 16, 33), (torch.bfloat16, 80, 16, 19),
     (torch.float16, 256, 9, 3),
+    (torch.bfloat16, 128, 145, 3), (torch.bfloat16, 128, 531, 2), (torch.float16, 64, 1100, 2),  # batches and their rest
+    (torch.float32, 128, 300, 2),
 ])
 def test_page_metadata_forms(dev, dtype, D, page, P):
     """Means and bounds are the oracle's bit for bit in both forms and into an
