@@ -309,7 +309,9 @@ int halo_chunk_means(const void* k, int64_t k_stride_b, int64_t k_stride_h, int6
  *   (:238-263); otherwise the raw attn.
  * Top-k order: score descending, then chunk index ascending; the k chosen
  * indices are written ascending to idx_out[s*k + j] (-1 when fewer than k are
- * eligible); raw/final scores to score_out[s*n_elig + i] when non-NULL.  When
+ * eligible); raw/final scores to score_out[s*n_elig + i] when non-NULL (large
+ * selections keep their raw scores there between two launches, so calls that
+ * may overlap need score buffers of their own).  When
  * `table` is non-NULL, descriptor catalog[s*catalog_stride + p] of each chosen
  * chunk p is copied to table[s*table_stride + table_slot0 + j] (an empty
  * descriptor, T_c = 0, fills unused slots), so a following halo_decode_attn

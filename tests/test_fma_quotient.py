@@ -1,4 +1,4 @@
-"""The KIVI quantiser (halo_amd/csrc/kivi.hip, kivi_code_fma) forms the
+"""The KIVI quantiser (halo_amd/csrc/kivi.hip, kivi_code_pair) forms the
 quotient (x - zero) / scale as q = d * (1/s) plus one FMA correction
 instead of a division.  This runs the exhaustive host check
 (tests/native/fma_quotient_check.c): for every pair of fp16 values, and
