@@ -35,7 +35,8 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
                       stream=None):
     """q (B, H, T_q, D) bf16, fp16 or fp32; chunks (B, H_kv, T_c, D) of the same dtype.
     Returns out (B, H, T_q, D) in ``out_dtype`` (default q.dtype) and, with
-    ``return_lse``, lse (B, H, T_q) fp32."""
+    ``return_lse``, lse (B, H, T_q) fp32.  With ``stream``, the inputs are
+    read and the results written there."""
     L = nat.lib()
     if q.dim() != 4:
         raise AssertionError(f"q must be (B, H, T_q, D), got {tuple(q.shape)}")
@@ -50,22 +51,22 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
     H_kv = chunks[0].k.shape[-3]
     if H % H_kv:
         raise AssertionError(f"head count mismatch: q has {H}, kv has {H_kv}")
-    q = _aligned_q(q)
-    qs_b, qs_h, qs_t = (st if n > 1 else 0 for st, n in zip(q.stride()[:3], q.shape)) if q.dtype == torch.float32 \
-        else q.stride()[:3]
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     T_all = sum([c.T for c in chunks])
     if q_start is None:
         q_start = T_all - T_q
     descs, keep = pack_descs(chunks, B=B, H_kv=H_kv, D=D, dtype=q.dtype)
-    # The uploads and the launch share one stream (the caller's, or the
-    # current one), so the kernel sees the tables; the tables are freed into
-    # torch's stream-ordered caching allocator on that stream.  q_start gets
+    # A copy of q, the uploads and the launch share one stream (the caller's,
+    # or the current one), so the kernel sees them; copy and tables are freed
+    # into torch's stream-ordered caching allocator on that stream.  q_start gets
     # there without a blocking copy (a pageable host-to-device copy would
     # hold the host until the stream drains); a plain number goes behind the
     # descriptors in their copy (a fill of its own was 4 us of host and 2-4 us
     # of GPU time in front of every call).  The caller owns the K/V.
     with torch.cuda.stream(stream) if stream is not None else _nullctx():
+        q = _aligned_q(q)
+        qs_b, qs_h, qs_t = (st if n > 1 else 0 for st, n in zip(q.stride()[:3], q.shape)) if q.dtype == torch.float32 \
+            else q.stride()[:3]
         if torch.is_tensor(q_start):
             if q_start.device.type != "cuda":
                 q_start = _to_device(q_start.to(torch.int64).reshape(-1).expand(B).numpy(), q.device)
@@ -143,10 +144,9 @@ def _prefill_fp32_rows(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale, q_
         starts = [int(q_start)] * B
     if len(starts) != B:
         raise AssertionError(f"q_start must have B={B} entries")
-    out = torch.empty((B, H, T_q, D), device=q.device, dtype=out_dtype or q.dtype)
-    lse = torch.empty((B, H, T_q), device=q.device, dtype=torch.float32) if return_lse else None
-    ctx = torch.cuda.stream(stream) if stream is not None else _nullctx()
-    with ctx:
+    with torch.cuda.stream(stream) if stream is not None else _nullctx():
+        out = torch.empty((B, H, T_q, D), device=q.device, dtype=out_dtype or q.dtype)
+        lse = torch.empty((B, H, T_q), device=q.device, dtype=torch.float32) if return_lse else None
         for b in range(B):
             rows = []
             for c in chunks:

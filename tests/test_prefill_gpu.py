@@ -83,3 +83,31 @@ def test_prefill_fp32_runs_on_the_decode_path(dev):
                                                           ChunkRef(kd[:, :, 64:], vd[:, :, 64:], 64, True)])
     want, _ = A.prefill_f64(q, k, v, scale=1 / math.sqrt(64), q_start=80 - 16)
     assert np.abs(out.cpu().numpy() - want).max() <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_prefill_on_a_side_stream(dev, dtype):
+    """A q that has to be copied for its alignment, made on a side stream and
+    passed with ``stream=``: the copy is ordered behind it and in front of the
+    kernels, whatever the current stream does."""
+    from halo_amd.decode import ChunkRef
+    from halo_amd.prefill import prefill_attention
+    rng = np.random.default_rng(5)
+    q, k, v = (round_to(rng.standard_normal(s, dtype=np.float32), dtype)
+               for s in ((1, 4, 40, 64), (1, 2, 104, 64), (1, 2, 104, 64)))
+    td = {**TDT, "float32": torch.float32}[dtype]
+    qh, kd, vd = (torch.from_numpy(a).to(dev).to(td) for a in (q, k, v))
+    wide = torch.zeros((1, 4, 40, 128), device=dev, dtype=td)
+    chunks = [ChunkRef(kd[:, :, :64], vd[:, :, :64], 0, False), ChunkRef(kd[:, :, 64:], vd[:, :, 64:], 64, True)]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        busy = torch.randn((2048, 2048), device=dev)
+        for _ in range(8):
+            busy = busy @ busy * 1e-3
+        wide[..., ::2] = qh
+    out, lse = prefill_attention(wide[..., ::2], chunks, q_start=64, return_lse=True, stream=side)
+    side.synchronize()
+    want, wl = A.prefill_f64(q, k, v, scale=1 / 8, q_start=64)
+    assert np.abs(out.float().cpu().numpy() - want).max() <= (1e-5 if dtype == "float32" else 2e-2)
+    assert np.abs(lse.cpu().numpy() - wl).max() <= 1e-5 * max(1.0, np.abs(wl).max())
