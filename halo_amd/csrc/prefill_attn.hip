@@ -33,16 +33,18 @@
 // Workgroups of one KV group run on one XCD (they share its L2), the ones with
 // the longest causal extent first.
 //
-// Calls whose rows give fewer workgroups than CUs leave the chip idle (512
-// rows x 32/8 heads: 64 of 256; the time is that of one workgroup's walk over
-// all keys).  There the walk is cut into n_split runs of key tiles, one
-// workgroup each, and prefill_merge_kernel folds the fp32 partials
-// (halo_prefill_splits holds the rule).  Per call, kernels only, bf16:
+// Calls whose rows give fewer workgroups than CUs, or a last round of few,
+// leave the chip idle (512 rows x 32/8 heads: 64 of 256; the time is that of
+// one workgroup's walk over all keys).  There the walk is cut into n_split runs
+// of key tiles, one workgroup each, and prefill_merge_kernel folds the fp32
+// partials (halo_prefill_splits holds the rule).  Per call, kernels only, bf16:
 //   512 rows over 8192 + 512 keys, 32/8 x 128:    238.6 us -> 90.4 us (4 splits)
 //   64 rows over 8192 + 64 keys, 32/8 x 128:      214.7 us -> 33.5 us (22)
 //   2 x 137 rows over 3000 + 137, 16/4 x 64, f16:  66.7 us -> 24.0 us (10)
-// The partials cost 2 x 4 bytes of traffic per output element and split, which
-// is why the rule stops at one workgroup per CU instead of cutting further.
+//   2304 rows over 32768 + 2304, 32/8 x 128 (288 workgroups): 1898 us -> 1273 (6)
+// The partials cost 2 x 4 bytes of traffic and 4 of workspace per output
+// element and split, which is what ends the cutting: the first in the rule's
+// model, the second by kPfMaxPartials.
 
 #include <type_traits>
 
@@ -966,6 +968,13 @@ int64_t prefill_units(int dtype, int B, int H, int H_kv, int T_q, int64_t* n_wg)
 }
 
 constexpr int kPfMaxSplit = 32;
+// Partials of the splits that are chosen here.  A call without splits takes no
+// workspace, so one that fits beside a large cache should not need much: 219 MiB
+// give the 288 workgroups of 2304 rows over 32768 keys their 6 splits, and more
+// workgroups need fewer (520 of 4100 rows: 2991 us unsplit, 2538 with the 3 that
+// fit, 2411 with 6 in 396 MiB; 1056 of 8392 rows over 65536: 10.65 ms unsplit,
+// which is all that fits, 9.29 with 5 in 670 MiB).
+constexpr int64_t kPfMaxPartials = 256ll << 20;
 
 // bytes of one wave's partial: 32 rows x D fp32 and 32 (m, l) pairs
 int64_t prefill_part_bytes(int D) { return 32ll * D * 4 + 32 * 8; }
@@ -976,11 +985,13 @@ int64_t prefill_part_bytes(int D) { return 32ll * D * 4 + 32 * 8; }
 // 8-wave workgroup per CU, each `mean` tiles at the measured time of a 64-key
 // tile (1.75 us at D = 128, 1.2 us at D = 64, every CU busy) plus prologue and
 // epilogue, or the longest workgroup alone; a split call adds the merge launch
-// and the partials written and read at 4 TB/s.  Against a sweep of 1 to 32
-// splits over 17 shapes (8 to 2500 rows, 0 to 16384 prior keys, 64 to 560
-// units) the choice was the fastest or within 5 % of it, but for one
-// (256 rows over 2048 keys 37.5 us for 35.6 us).  fp32: 32-key tiles, 3.1 and
-// 5.5 us with one 4-wave workgroup on a CU, 4.4 and 9.2 us each with two.
+// and the partials written and read at 4 TB/s.  Against sweeps of 1 to 32
+// splits over 28 shapes (8 to 8392 rows, 0 to 131072 prior keys, 64 to 2080
+// units) the model's choice was the fastest or within 5 % of it, but for one
+// (256 rows over 2048 keys 37.5 us for 35.6 us); the partials have to fit
+// kPfMaxPartials.  fp32: 32-key tiles, 3.1 and 5.5 us with one 4-wave workgroup
+// on a CU, 4.4 and 9.2 us each with two; fastest or within 3 % over 6 shapes
+// (512 to 4100 rows, 2048 and 8192 keys).
 extern "C" int halo_prefill_splits(int dtype, int B, int H, int H_kv, int T_q, int D, int64_t keys, int64_t causal_keys) {
   if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || T_q <= 0 || D <= 0 || keys <= 0) return 1;
   int64_t n_wg;
@@ -991,9 +1002,10 @@ extern "C" int halo_prefill_splits(int dtype, int B, int H, int H_kv, int T_q, i
   const double longest = (double)(keys + bk - 1) / bk;
   const int64_t tri = causal_keys < T_q ? causal_keys : T_q;
   const double mean = longest - 0.5 * (double)tri / bk;
+  const int64_t part = units * nw * prefill_part_bytes(D);
   double best = 0;
   int best_s = 1;
-  for (int s = 1; s <= kPfMaxSplit && s <= (int)longest; ++s) {
+  for (int s = 1; s <= kPfMaxSplit && s <= (int)longest && (s == 1 || s * part <= kPfMaxPartials); ++s) {
     const bool pairs = f32 && units * s > 256;  // fp32: two 4-wave workgroups per CU
     const int slots = pairs ? 512 : 256;
     const double tile_us = f32 ? (pairs ? (D == 128 ? 9.2 : 4.4) : (D == 128 ? 5.5 : 3.1)) : (D == 128 ? 1.75 : 1.2);
@@ -1001,7 +1013,7 @@ extern "C" int halo_prefill_splits(int dtype, int B, int H, int H_kv, int T_q, i
     const double chip = rounds * (mean / s * tile_us + fixed_us);
     const double one = std::ceil(longest / s) * tile_us + fixed_us;
     double us = chip > one ? chip : one;
-    if (s > 1) us += 5.0 + (double)s * (double)(units * nw * prefill_part_bytes(D)) * 2.0 / 4.0e6;
+    if (s > 1) us += 5.0 + (double)s * (double)part * 2.0 / 4.0e6;
     if (s == 1 || us < best) {
       best = us;
       best_s = s;

@@ -86,7 +86,10 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
         dt = nat.dtype_code(q.dtype)
         n_split = L.halo_prefill_splits(dt, B, H, H_kv, T_q, D, T_all, sum([c.T for c in chunks if c.causal]))
         ws_bytes = L.halo_prefill_workspace_size(dt, B, H, H_kv, T_q, D, n_split)
-        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
+        try:
+            ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
+        except torch.OutOfMemoryError:  # the unsplit walk needs none
+            n_split, ws_bytes, ws = 1, 0, None
         nat.check(L.halo_prefill_attn_split(
             q.data_ptr(), qs_b, qs_h, qs_t, dt, B, H, H_kv, T_q, D,
             starts, d_descs.data_ptr(), len(chunks), scale,

@@ -265,14 +265,15 @@ int halo_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, int
 /*
  * The same attention with the keys of every query block cut into n_split
  * consecutive runs of 64-row tiles, one workgroup each, and a merge of the
- * fp32 partials (n_split 1: halo_prefill_attn, no workspace).  For calls with
- * too few query rows to fill the GPU.  Also takes HALO_F32 queries and chunks
+ * fp32 partials (n_split 1: halo_prefill_attn, no workspace).  For calls whose
+ * query rows do not fill the GPU or leave its last round nearly empty.  Also takes HALO_F32 queries and chunks
  * (fp32 products and sums on the matrix cores; rows, head and batch strides of
  * q, K and V 16-byte aligned, row strides of K and V at least D and below 2^22
  * elements).  `workspace` (16-byte aligned) holds at
  * least halo_prefill_workspace_size bytes; halo_prefill_splits returns the
  * n_split (1 to 32) expected to be the fastest over `keys` attended rows of
- * which `causal_keys` are in causal chunks.
+ * which `causal_keys` are in causal chunks, among those whose workspace is at
+ * most 256 MiB.
  */
 int halo_prefill_splits(int dtype, int B, int H, int H_kv, int T_q, int D, int64_t keys, int64_t causal_keys);
 size_t halo_prefill_workspace_size(int dtype, int B, int H, int H_kv, int T_q, int D, int n_split);

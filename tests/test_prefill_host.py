@@ -92,3 +92,39 @@ def test_device_work_is_on_the_given_stream(host, monkeypatch, dtype, direct, q_
     with _Writes(state) as seen:
         P.prefill_attention(q, [_chunk(dtype)], return_lse=True, stream=object())
     assert seen.outside == []
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_split_workspace_is_bounded(dtype):
+    """The library's choice of key splits takes at most 256 MiB of partials,
+    whatever the rows and keys (2304 and 4100 rows are just past a round of
+    workgroups in 16 and 32 bits), and does split where that is little."""
+    from halo_amd import _native as nat
+    L, dt = nat._load(), nat.dtype_code(dtype)
+    split = 0
+    for B in (1, 2, 4, 16):
+        for H, H_kv, D in ((32, 8, 128), (28, 4, 128), (16, 4, 64), (8, 8, 64)):
+            for T_q in (1, 137, 512, 1100, 2080, 2304, 4100, 4160, 8392, 33000):
+                for prior in (0, 2048, 32768, 131072, 1 << 20):
+                    s = L.halo_prefill_splits(dt, B, H, H_kv, T_q, D, prior + T_q, T_q)
+                    assert L.halo_prefill_workspace_size(dt, B, H, H_kv, T_q, D, s) <= 256 << 20
+                    split += s > 1
+    assert split > 100
+
+
+def test_call_without_memory_for_the_partials_runs_unsplit(host, monkeypatch):
+    from halo_amd import prefill as P
+    host.n_split, host.ws_bytes = 4, 1 << 20
+    real = torch.empty
+
+    def empty(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return real(*a, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    P.prefill_attention(torch.zeros((1, 4, 8, 64), dtype=torch.bfloat16), [_chunk(torch.bfloat16)])
+    assert host.attn_args[-4:-1] == (1, None, 0)
+    monkeypatch.setattr(torch, "empty", real)
+    P.prefill_attention(torch.zeros((1, 4, 8, 64), dtype=torch.bfloat16), [_chunk(torch.bfloat16)])
+    assert host.attn_args[-4] == 4 and host.attn_args[-2] == 1 << 20
