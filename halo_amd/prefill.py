@@ -52,9 +52,8 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
     if H % H_kv:
         raise AssertionError(f"head count mismatch: q has {H}, kv has {H_kv}")
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    T_all = sum([c.T for c in chunks])
     if q_start is None:
-        q_start = T_all - T_q
+        q_start = sum([c.T for c in chunks]) - T_q
     descs, keep = pack_descs(chunks, B=B, H_kv=H_kv, D=D, dtype=q.dtype)
     # A copy of q, the uploads and the launch share one stream (the caller's,
     # or the current one), so the kernel sees them; copy and tables are freed
@@ -84,7 +83,7 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
         out = torch.empty((B, H, T_q, D), device=q.device, dtype=out_dtype or q.dtype)
         lse = torch.empty((B, H, T_q), device=q.device, dtype=torch.float32) if return_lse else None
         dt = nat.dtype_code(q.dtype)
-        n_split = L.halo_prefill_splits(dt, B, H, H_kv, T_q, D, T_all, sum([c.T for c in chunks if c.causal]))
+        n_split = L.halo_prefill_splits(dt, B, H, H_kv, T_q, D, *_longest_walk(chunks))
         ws_bytes = L.halo_prefill_workspace_size(dt, B, H, H_kv, T_q, D, n_split)
         try:
             ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
@@ -97,6 +96,23 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
             nat.ptr(lse), n_split, nat.ptr(ws), ws_bytes, nat.stream_ptr(stream)), "halo_prefill_attn_split")
     del keep
     return (out, lse) if return_lse else out
+
+
+def _longest_walk(chunks: Sequence[ChunkRef]) -> tuple[int, int]:
+    """(keys, keys in causal chunks) of the batch row that attends most keys."""
+    keys = causal = 0
+    own: dict = {}
+    for c in chunks:
+        n = c.T
+        if c.batch < 0:
+            keys += n
+            if c.causal:
+                causal += n
+        else:
+            k, d = own.get(c.batch, (0, 0))
+            own[c.batch] = (k + n, d + n if c.causal else d)
+    k, d = max(own.values(), default=(0, 0))
+    return keys + k, causal + d
 
 
 def _aligned_q(q: torch.Tensor) -> torch.Tensor:

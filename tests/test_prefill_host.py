@@ -128,3 +128,19 @@ def test_call_without_memory_for_the_partials_runs_unsplit(host, monkeypatch):
     monkeypatch.setattr(torch, "empty", real)
     P.prefill_attention(torch.zeros((1, 4, 8, 64), dtype=torch.bfloat16), [_chunk(torch.bfloat16)])
     assert host.attn_args[-4] == 4 and host.attn_args[-2] == 1 << 20
+
+
+@pytest.mark.parametrize("batches,causal,want", [
+    ((-1, -1, -1), (False, False, True), (96, 32)),   # every row reads every chunk
+    ((0, 1, 2), (True, True, True), (32, 32)),        # one chunk a row
+    ((0, 0, 2), (False, True, True), (64, 32)),       # the row with most keys
+    ((-1, 1, 1), (False, False, True), (96, 32)),     # shared rows and a row's own
+    ((-1, 0, -1), (False, True, True), (96, 64)),
+])
+def test_split_rule_gets_the_longest_walk(host, batches, causal, want):
+    """The keys of one batch row and not those of the whole list: chunks of
+    other rows are not part of a workgroup's walk."""
+    from halo_amd import prefill as P
+    chunks = [_chunk(torch.bfloat16, B=3, batch=b, causal=c) for b, c in zip(batches, causal)]
+    P.prefill_attention(torch.zeros((3, 4, 8, 64), dtype=torch.bfloat16), chunks, q_start=0)
+    assert host.splits_args[-2:] == want
