@@ -54,6 +54,8 @@ def prefill_attention(q: torch.Tensor, chunks: Sequence[ChunkRef], *, scale: Opt
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     if q_start is None:
         q_start = sum([c.T for c in chunks]) - T_q
+    if q.dtype == torch.float32 and torch.is_tensor(q_start) and q_start.numel() not in (1, B):
+        raise AssertionError(f"q_start must have B={B} entries")
     descs, keep = pack_descs(chunks, B=B, H_kv=H_kv, D=D, dtype=q.dtype)
     # A copy of q, the uploads and the launch share one stream (the caller's,
     # or the current one), so the kernel sees them; copy and tables are freed

@@ -144,3 +144,14 @@ def test_split_rule_gets_the_longest_walk(host, batches, causal, want):
     chunks = [_chunk(torch.bfloat16, B=3, batch=b, causal=c) for b, c in zip(batches, causal)]
     P.prefill_attention(torch.zeros((3, 4, 8, 64), dtype=torch.bfloat16), chunks, q_start=0)
     assert host.splits_args[-2:] == want
+
+
+@pytest.mark.parametrize("q_start", [torch.zeros(3, dtype=torch.int64), torch.zeros(0, dtype=torch.int64)])
+@pytest.mark.parametrize("direct", [True, False])
+def test_fp32_q_start_of_the_wrong_length(host, monkeypatch, q_start, direct):
+    """Both fp32 forms refuse it by name."""
+    from halo_amd import prefill as P
+    monkeypatch.setattr(P, "_f32_direct", lambda q, chunks: direct)
+    q = torch.zeros((2, 4, 8, 64))
+    with pytest.raises(AssertionError, match="q_start must have B=2 entries"):
+        P.prefill_attention(q, [_chunk(torch.float32, B=2)], q_start=q_start)
