@@ -136,7 +136,7 @@ def _f32_direct(q: torch.Tensor, chunks: Sequence[ChunkRef]) -> bool:
         for t in (getattr(c, "k", None), getattr(c, "v", None)):
             if t is None or t.dim() != 4 or t.shape[0] != B or t.shape[-1] != D or t.dtype != torch.float32:
                 return False
-            if getattr(c, "batch", -1) >= 0 or t.stride(-1) != 1 or t.data_ptr() % 16:
+            if getattr(c, "batch", 0) >= 0 or t.stride(-1) != 1 or t.data_ptr() % 16:
                 return False
             sb, sh, st = t.stride()[:3]
             if (t.shape[0] > 1 and sb % 4) or (t.shape[1] > 1 and sh % 4) or st % 4 or not D <= st < 1 << 22:

@@ -155,3 +155,14 @@ def test_fp32_q_start_of_the_wrong_length(host, monkeypatch, q_start, direct):
     q = torch.zeros((2, 4, 8, 64))
     with pytest.raises(AssertionError, match="q_start must have B=2 entries"):
         P.prefill_attention(q, [_chunk(torch.float32, B=2)], q_start=q_start)
+
+
+def test_fp32_chunks_without_a_batch():
+    """The row form needs k, v, chunk_start and causal of a chunk and no more:
+    an object with just these stays with it."""
+    from types import SimpleNamespace
+
+    from halo_amd.prefill import _f32_direct
+    q = SimpleNamespace(is_cuda=True, shape=(1, 4, 8, 64))
+    k = torch.zeros((1, 2, 32, 64))
+    assert not _f32_direct(q, [SimpleNamespace(k=k, v=k, chunk_start=0, causal=True)])
