@@ -1078,9 +1078,10 @@ extern "C" int halo_prefill_attn_split(const void* q, int64_t q_stride_b, int64_
   p.descs = descs;
   p.n_desc = n_desc;
   p.scale2 = (float)((double)scale * 1.4426950408889634);
-  // a masked score is an infinity times the scale: a zero scale would make it NaN,
-  // and the smallest normal number leaves every finite score at 2^0 all the same
-  if (dtype == HALO_F32 && p.scale2 == 0.f) p.scale2 = 1.17549435e-38f;
+  // a masked score is an infinity times the scale: a zero scale would make it NaN.
+  // The smallest subnormal, 2^-149, leaves scores below 2^125 at 2^0 and the fp32
+  // maximum within 3.3e-7 of it
+  if (dtype == HALO_F32 && p.scale2 == 0.f) p.scale2 = 0x1p-149f;
   p.out = out;
   p.o_stride_b = out_stride_b;
   p.o_stride_h = out_stride_h;

@@ -110,6 +110,23 @@ def test_fp32_call(dev, T_q, prior, D, scale):
     assert torch.equal(out2[:, 3:, -1, :5], out[:, 3:, -1, :5])
 
 
+@gpu
+def test_fp32_zero_scale_of_large_scores(dev):
+    """A zero scale weighs every visible key alike, however large the scores:
+    of up to 1e38 here, 3e-7 relative in a weight at the fp32 maximum."""
+    from halo_amd.decode import ChunkRef
+    from halo_amd.prefill import prefill_attention
+    rng = np.random.default_rng(8)
+    q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((1, 4, 40, 64), (1, 2, 140, 64), (1, 2, 140, 64)))
+    k *= np.float32(2e36)
+    qt, kt, vt = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    chunks = [ChunkRef(kt[:, :, :100], vt[:, :, :100], 0, False), ChunkRef(kt[:, :, 100:], vt[:, :, 100:], 100, True)]
+    out, lse = prefill_attention(qt, chunks, scale=0.0, return_lse=True)
+    want, wl = A.prefill_f64(q, k, v, scale=0.0, q_start=100)
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5
+    assert np.abs(lse.cpu().numpy() - wl).max() <= 1e-5
+
+
 def test_fp32_route():
     """Chunks that the matrix kernel does not read stay on the row-by-row form."""
     from halo_amd.decode import ChunkRef
