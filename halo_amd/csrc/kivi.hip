@@ -162,7 +162,15 @@ __device__ __forceinline__ void kivi_code_pair(float& a, float& b, const float4&
   a = __builtin_amdgcn_fmed3f(rintf(a), 0.f, qmax);
   b = __builtin_amdgcn_fmed3f(rintf(b), 0.f, qmax);
 }
-// min(a, x, y) and max(a, x, y), NaN dropped, in one operation each
+// min(a, x, y) and max(a, x, y), NaN dropped, in one operation each.  With the
+// IEEE bit of the mode register set, as a kernel begins, a signalling NaN (a bf16
+// element can be one: its conversion is a shift) comes back as a quiet one and
+// takes `a` with it; drop_all_nan clears the bit.  Quieting every element
+// instead costs an operation each.
+__device__ __forceinline__ void drop_all_nan() {
+  constexpr int kMode = 1, kIeeeBit = 9;  // hwreg(HW_REG_MODE, 9, 1)
+  __builtin_amdgcn_s_setreg(kMode | kIeeeBit << 6, 0);
+}
 __device__ __forceinline__ float kmin3(float a, float x, float y) {
   float r;
   asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(x), "v"(y));
@@ -273,6 +281,7 @@ __global__ void __launch_bounds__(256) kivi_quantize_kernel(KiviQuantParams P) {
   __shared__ float s_vmn[2][G * NG], s_vmx[2][G * NG];
   __shared__ __align__(16) float4 s_kp[KP];  // kivi_code_params per channel
   __shared__ __align__(16) float4 s_vp[G * NG];
+  drop_all_nan();
   const int tid = threadIdx.x;
   const int j = blockIdx.x % P.n_blk;
   const int bh = blockIdx.x / P.n_blk;

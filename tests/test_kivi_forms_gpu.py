@@ -56,3 +56,24 @@ def test_quantise_and_dequantise_forms(dev, dtype, D, n, bits):
     ke = torch.empty(kt.numel() + 1, device=dev, dtype=kt.dtype)[1:].view(kt.shape)
     ke.copy_(kt)
     assert torch.equal(kivi.quantize(ke, vt, bits=bits), blocks)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_signalling_nan(dev, D, bits):
+    """bf16 NaN elements get code 0 and leave the range of their group to the
+    others, quiet or signalling alike."""
+    from halo_amd import kivi
+    rng = np.random.default_rng(bits)
+    x = torch.from_numpy(rng.standard_normal((1, 2, 96, D), dtype=np.float32)).to(dev).to(torch.bfloat16)
+    blocks = []
+    for nan in (0x7FC1, 0x7F81, 0xFF82 - 0x10000):
+        y = x.clone()
+        y.view(torch.int16)[:, :, 5::7, 3::5] = nan
+        y.view(torch.int16)[:, 1, 32:64:2, 9] = nan
+        blocks.append(kivi.quantize(y, y.flip(2).contiguous(), bits=bits))
+    assert torch.equal(blocks[0], blocks[1]) and torch.equal(blocks[0], blocks[2])
+    kd, vd = kivi.dequantize(blocks[0], D=D, dtype=torch.bfloat16, bits=bits)
+    assert not kd.isnan().any() and not vd.isnan().any()
+    keep = ~y.isnan()  # the codes of the numbers: within half a step of their group's range, which is below 10
+    assert (kd - y).abs()[keep].max().item() <= 10 / (2 ** bits - 1) / 2 + 0.05
