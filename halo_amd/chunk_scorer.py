@@ -54,7 +54,7 @@ def score_topk(q: torch.Tensor, kmean: torch.Tensor, eligible: torch.Tensor, k: 
                catalog: Optional[torch.Tensor] = None, table: Optional[torch.Tensor] = None,
                table_stride: int = 0, table_slot0: int = 0, catalog_stride: int = 0,
                idx_out: Optional[torch.Tensor] = None, score_out: Optional[torch.Tensor] = None,
-               staging: Optional[tuple] = None):
+               staging: Optional[tuple] = None, workspace: Optional[torch.Tensor] = None):
     """Score eligible chunks and pick the top ``k``.
 
     q (B, H, D) or (B, H, 1, D); kmean (B, H_kv, P, D) in q's dtype;
@@ -64,8 +64,10 @@ def score_topk(q: torch.Tensor, kmean: torch.Tensor, eligible: torch.Tensor, k: 
     chosen descriptors are copied into the table on the device.
     ``staging`` = (residency int32 tensor, slot catalog uint8 tensor,
     n_slots, res_out int32 tensor): chosen chunks held by an HBM staging
-    slot are written to the table with the slot's addresses
-    (``halo_chunk_score_topk_staged``; raw scores only)."""
+    slot are written to the table with the slot's addresses (raw scores only).
+    ``workspace`` (fp32, (n_sel, n_elig)) holds the raw scores of a large
+    selection between its two launches, so calls that may overlap need one
+    each; by default it is a buffer of this call's own."""
     L = nat.lib()
     q3 = q.squeeze(2) if q.dim() == 4 else q
     B, H, D = q3.shape
@@ -85,25 +87,22 @@ def score_topk(q: torch.Tensor, kmean: torch.Tensor, eligible: torch.Tensor, k: 
     eligible = eligible.contiguous()
     if idx_out is None:
         idx_out = torch.empty((n_sel, k), device=q3.device, dtype=torch.int32)
-    if score_out is None:
-        score_out = torch.empty((n_sel, max(n_elig, 1)), device=q3.device, dtype=torch.float32)
+    if workspace is None or score_out is None:
+        own = torch.empty((n_sel, max(n_elig, 1)), device=q3.device, dtype=torch.float32)
+        workspace = own if workspace is None else workspace
+        score_out = own if score_out is None else score_out
+    if workspace.dtype != torch.float32 or not workspace.is_contiguous() or workspace.numel() < n_sel * n_elig:
+        raise AssertionError(f"workspace must be contiguous float32 of {n_sel * n_elig} entries")
     if catalog is not None and catalog_stride == 0 and per_row:
         catalog_stride = catalog.numel() // 88 // n_sel
+    res = (None, None, 0, None)
     if staging is not None:
         if normalize or table is None:
             raise AssertionError("the staged selection writes a table and uses raw scores")
-        res, scat, n_slots, res_out = staging
-        nat.check(L.halo_chunk_score_topk_staged(
-            q3.data_ptr(), q3.stride(0), q3.stride(1), nat.dtype_code(q3.dtype),
-            B, H, H_kv, D,
-            kmean.data_ptr(), kmean.stride(0), kmean.stride(1), kmean.stride(2),
-            eligible.data_ptr(), elig_stride, nat.ptr(n_elig_per_sel), n_elig, int(k), int(per_row),
-            idx_out.data_ptr(), score_out.data_ptr(),
-            nat.ptr(catalog), catalog_stride or n_elig, nat.ptr(table), table_stride, table_slot0,
-            res.data_ptr(), scat.data_ptr(), int(n_slots), res_out.data_ptr(), nat.stream_ptr()),
-            "halo_chunk_score_topk_staged")
-        return idx_out, score_out
-    nat.check(L.halo_chunk_score_topk(
+        r, scat, n_slots, res_out = staging
+        res = (r.data_ptr(), scat.data_ptr(), int(n_slots), res_out.data_ptr())
+        catalog_stride = catalog_stride or n_elig
+    nat.check(L.halo_chunk_score_topk_ws(
         q3.data_ptr(), q3.stride(0), q3.stride(1), nat.dtype_code(q3.dtype),
         B, H, H_kv, D,
         kmean.data_ptr(), kmean.stride(0), kmean.stride(1), kmean.stride(2),
@@ -111,7 +110,8 @@ def score_topk(q: torch.Tensor, kmean: torch.Tensor, eligible: torch.Tensor, k: 
         idx_out.data_ptr(), score_out.data_ptr(),
         nat.ptr(catalog), catalog_stride, nat.ptr(table), table_stride, table_slot0,
         int(normalize), float(alpha), float(beta), float(gamma), int(refresh_window), int(sink_pages),
-        int(P_total if P_total is not None else P), nat.stream_ptr()), "halo_chunk_score_topk")
+        int(P_total if P_total is not None else P), *res, workspace.data_ptr(), nat.stream_ptr()),
+        "halo_chunk_score_topk_ws")
     return idx_out, score_out
 
 

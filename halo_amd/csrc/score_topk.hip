@@ -189,7 +189,8 @@ struct ScoreParams {
   const halo_chunk_desc* slot_catalog;
   int n_slots;
   int32_t* res_out;
-  int qvec;  // q rows are 16-byte aligned (score_pages_kernel)
+  int qvec;    // q rows are 16-byte aligned (score_pages_kernel)
+  float* raw;  // (n_sel, n_elig) raw scores between score_pages_kernel and the selection
 };
 
 constexpr int kMaxElig = 1024;
@@ -238,7 +239,7 @@ __device__ __forceinline__ void select_ascending(const float* s_score, int n, in
   }
 }
 
-// Raw scores of many pages, spread over the GPU: score_out[sel, i] = max over
+// Raw scores of many pages, spread over the GPU: raw[sel, i] = max over
 // (row, head) of qg . kbar, in the slice order of score_topk_kernel.  G = D/16
 // lanes per page, lane c on slice c, so a wave reads whole rows of 64/G2 pages;
 // the four waves of a workgroup take the (row, head) pairs in turn and meet in
@@ -286,13 +287,13 @@ __global__ void __launch_bounds__(256) score_pages_kernel(ScoreParams P, int til
   __syncthreads();
   const int t = threadIdx.x;
   if (t < PPW && tile * PPW + t < n)
-    P.score_out[(int64_t)sel * P.n_elig + tile * PPW + t] =
+    P.raw[(int64_t)sel * P.n_elig + tile * PPW + t] =
         fmaxf(fmaxf(s_best[0][t], s_best[1][t]), fmaxf(s_best[2][t], s_best[3][t]));
 }
 
 // DC: the head dim when known at compile time (64, 128, 256: the dot-product
 // loops unroll and every load of a triple is issued before the first use),
-// 0 for any other multiple of 16 (runtime loops), -1: score_out holds the raw
+// 0 for any other multiple of 16 (runtime loops), -1: P.raw holds the raw
 // scores (score_pages_kernel) and only the combination and the top-k remain.
 template <int DT, int DC>
 __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
@@ -314,7 +315,7 @@ __global__ void __launch_bounds__(512) score_topk_kernel(ScoreParams P) {
   for (int i = tid; i < n; i += nthr) s_chunk[i] = elig[i];
   if constexpr (kGiven) {
     for (int i = tid; i < n; i += nthr) {
-      const float v = P.score_out[(int64_t)sel * P.n_elig + i];
+      const float v = P.raw[(int64_t)sel * P.n_elig + i];
       s_score[i] = v != v ? -INFINITY : v;
     }
     __syncthreads();
@@ -649,7 +650,7 @@ static int score_topk_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h
                                      int normalize, float alpha, float beta, float gamma,
                                      int refresh, int sink_pages, int P_total,
                                      const int32_t* residency, const halo_chunk_desc* slot_catalog, int n_slots,
-                                     int32_t* res_out, void* stream) {
+                                     int32_t* res_out, float* workspace, void* stream) {
   HALO_CHECK_ARG(q && kmean && eligible, "null pointer");
   HALO_CHECK_ARG(residency == nullptr || (slot_catalog != nullptr && n_slots >= 1 && table != nullptr),
                  "staging needs slot_catalog, n_slots >= 1 and a table");
@@ -710,12 +711,13 @@ static int score_topk_impl(const void* q, int64_t q_stride_b, int64_t q_stride_h
   const int es = elem_size(dtype);
   p.qvec = reinterpret_cast<uintptr_t>(q) % 16 == 0 && (q_stride_b * es) % 16 == 0 && (q_stride_h * es) % 16 == 0;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // Scores on their own grid, held by score_out until the selection reads
+  // Scores on their own grid, held by the workspace until the selection reads
   // them, where one CU would walk the means for longer than a launch costs.
   // Own grid / one workgroup, at 8 heads x 128 bf16: 16 pages 8.3 / 8.4 us, 32
   // 8.9 / 9.1, 64 8.8 / 10.8, 512 11.8 / 38; at 4 heads x 64: 64 pages 7.3 / 6.6,
   // 128 7.6 / 7.8, 512 9.9 / 15.3.
-  if (score_out != nullptr && (int64_t)n_elig * nrows * H_kv * D >= 32768) {
+  p.raw = workspace;
+  if (workspace != nullptr && (int64_t)n_elig * nrows * H_kv * D >= 32768) {
     const int G = D / 16;
     const int G2 = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : G <= 8 ? 8 : 16;
     const int tiles = (n_elig + 64 / G2 - 1) / (64 / G2);
@@ -766,7 +768,7 @@ extern "C" int halo_chunk_score_topk(const void* q, int64_t q_stride_b, int64_t 
   return score_topk_impl(q, q_stride_b, q_stride_h, dtype, B, H, H_kv, D, kmean, km_stride_b, km_stride_h,
                          km_stride_p, eligible, elig_stride, n_elig_per_sel, n_elig, k, per_row, idx_out, score_out,
                          catalog, catalog_stride, table, table_stride, table_slot0, normalize, alpha, beta, gamma,
-                         refresh, sink_pages, P_total, nullptr, nullptr, 0, nullptr, stream);
+                         refresh, sink_pages, P_total, nullptr, nullptr, 0, nullptr, nullptr, stream);
 }
 
 extern "C" int halo_chunk_score_topk_staged(const void* q, int64_t q_stride_b, int64_t q_stride_h, int dtype,
@@ -784,5 +786,25 @@ extern "C" int halo_chunk_score_topk_staged(const void* q, int64_t q_stride_b, i
   return score_topk_impl(q, q_stride_b, q_stride_h, dtype, B, H, H_kv, D, kmean, km_stride_b, km_stride_h,
                          km_stride_p, eligible, elig_stride, n_elig_per_sel, n_elig, k, per_row, idx_out, score_out,
                          catalog, catalog_stride, table, table_stride, table_slot0, 0, 1.f, 0.f, 0.f, 64, 0, 1,
-                         residency, slot_catalog, n_slots, res_out, stream);
+                         residency, slot_catalog, n_slots, res_out, nullptr, stream);
+}
+
+extern "C" int halo_chunk_score_topk_ws(const void* q, int64_t q_stride_b, int64_t q_stride_h, int dtype,
+                                        int B, int H, int H_kv, int D,
+                                        const void* kmean, int64_t km_stride_b, int64_t km_stride_h,
+                                        int64_t km_stride_p,
+                                        const int32_t* eligible, int64_t elig_stride,
+                                        const int32_t* n_elig_per_sel, int n_elig, int k, int per_row,
+                                        int32_t* idx_out, float* score_out,
+                                        const halo_chunk_desc* catalog, int64_t catalog_stride,
+                                        halo_chunk_desc* table, int64_t table_stride, int table_slot0,
+                                        int normalize, float alpha, float beta, float gamma,
+                                        int refresh, int sink_pages, int P_total,
+                                        const int32_t* residency, const halo_chunk_desc* slot_catalog,
+                                        int n_slots, int32_t* res_out, float* workspace, void* stream) {
+  HALO_CHECK_ARG(residency == nullptr || !normalize, "the staged selection uses raw scores");
+  return score_topk_impl(q, q_stride_b, q_stride_h, dtype, B, H, H_kv, D, kmean, km_stride_b, km_stride_h,
+                         km_stride_p, eligible, elig_stride, n_elig_per_sel, n_elig, k, per_row, idx_out, score_out,
+                         catalog, catalog_stride, table, table_stride, table_slot0, normalize, alpha, beta, gamma,
+                         refresh, sink_pages, P_total, residency, slot_catalog, n_slots, res_out, workspace, stream);
 }

@@ -117,7 +117,7 @@ class ColdStaging:
         self.top_k = lay0.top_k
         # fused layers select in the attention launch (halo_select_cfg);
         # unfused ones (beyond the fused selection's limits) run the staged
-        # scorer (halo_chunk_score_topk_staged) before the attention launch
+        # scorer (halo_chunk_score_topk_ws with residency) before the attention launch
         for li, lay in enumerate(self.layers):
             fused = getattr(lay, "select_cfg", None) is not None and getattr(lay, "fused", True)
             if not fused and not hasattr(lay, "staging"):

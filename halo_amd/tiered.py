@@ -7,7 +7,7 @@ Per step (fused mode, the default) this enqueues one
 query, take the chosen chunks' descriptors from the catalog and attend them,
 while the other workgroups attend the hot chunks; the split-K merge kernel
 then writes (out, lse).  Unfused mode (``fused=False``, or shapes beyond the
-in-kernel selection limits) enqueues ``halo_chunk_score_topk`` (which copies
+in-kernel selection limits) enqueues ``halo_chunk_score_topk_ws`` (which copies
 the chosen descriptors into the table's slots) followed by
 ``halo_decode_attn``.  Either way there is no host round trip, so a whole
 multi-layer decode step can be captured in one HIP graph.
@@ -124,11 +124,12 @@ class TieredDecodeLayer:
         return sum(c.T for c in self.hot) + self.top_k * per
 
     def select(self, q: torch.Tensor) -> None:
-        """Standalone selection (``halo_chunk_score_topk``): fills idx/scores
-        and the table's selection slots."""
+        """Standalone selection (``halo_chunk_score_topk_ws``): fills idx/scores
+        and the table's selection slots.  The scores are its workspace as well:
+        selections of one layer may not overlap anyway (they share the slots)."""
         score_topk(q, self.kmean, self.eligible, self.top_k, catalog=self.catalog,
                    table=self.plan.descs, table_slot0=self.slot0, idx_out=self.idx, score_out=self.scores,
-                   staging=self.staging)
+                   staging=self.staging, workspace=self.scores)
 
     def attend(self, q: torch.Tensor, *, scale: float, out: torch.Tensor, lse: Optional[torch.Tensor] = None,
                q_pos: Optional[torch.Tensor] = None) -> None:

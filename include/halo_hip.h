@@ -310,9 +310,7 @@ int halo_chunk_means(const void* k, int64_t k_stride_b, int64_t k_stride_h, int6
  *   (:238-263); otherwise the raw attn.
  * Top-k order: score descending, then chunk index ascending; the k chosen
  * indices are written ascending to idx_out[s*k + j] (-1 when fewer than k are
- * eligible); raw/final scores to score_out[s*n_elig + i] when non-NULL (large
- * selections keep their raw scores there between two launches, so calls that
- * may overlap need score buffers of their own).  When
+ * eligible); raw/final scores to score_out[s*n_elig + i] when non-NULL.  When
  * `table` is non-NULL, descriptor catalog[s*catalog_stride + p] of each chosen
  * chunk p is copied to table[s*table_stride + table_slot0 + j] (an empty
  * descriptor, T_c = 0, fills unused slots), so a following halo_decode_attn
@@ -358,6 +356,28 @@ int halo_chunk_score_topk_staged(const void* q, int64_t q_stride_b, int64_t q_st
                                  halo_chunk_desc* table, int64_t table_stride, int table_slot0,
                                  const int32_t* residency, const halo_chunk_desc* slot_catalog,
                                  int n_slots, int32_t* res_out, void* stream);
+
+/*
+ * Both of the above (residency NULL: halo_chunk_score_topk) with scratch for
+ * the raw scores: with a `workspace` of n_sel * n_elig floats a large
+ * selection is scored on a grid of its own and selected by a second launch.
+ * It may be score_out, where no other call that may overlap has that buffer;
+ * calls that may overlap need workspaces of their own.  NULL: one launch of
+ * one workgroup per selection, as above.  The results are the same.
+ */
+int halo_chunk_score_topk_ws(const void* q, int64_t q_stride_b, int64_t q_stride_h, int dtype,
+                             int B, int H, int H_kv, int D,
+                             const void* kmean, int64_t km_stride_b, int64_t km_stride_h,
+                             int64_t km_stride_p,
+                             const int32_t* eligible, int64_t elig_stride,
+                             const int32_t* n_elig_per_sel, int n_elig, int k, int per_row,
+                             int32_t* idx_out, float* score_out,
+                             const halo_chunk_desc* catalog, int64_t catalog_stride,
+                             halo_chunk_desc* table, int64_t table_stride, int table_slot0,
+                             int normalize, float alpha, float beta, float gamma,
+                             int refresh, int sink_pages, int P_total,
+                             const int32_t* residency, const halo_chunk_desc* slot_catalog,
+                             int n_slots, int32_t* res_out, float* workspace, void* stream);
 
 /*
  * Quest page metadata: channel-wise minima and maxima of `n_pages` pages of
