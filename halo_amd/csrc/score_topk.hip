@@ -15,6 +15,17 @@
 
 namespace halo {
 
+// fp16 means of two sums, each product rounded once, to fp16 (written out: left
+// to the compiler a product and its conversion are one or two roundings; the
+// wait state is the one between two writes of halves of a register).
+__device__ __forceinline__ uint32_t mean_f16(float lo, float hi, float inv) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %3, 0\n\ts_nop 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0"
+      : "=&v"(r)
+      : "v"(lo), "v"(hi), "v"(inv));
+  return r;
+}
+
 // ---------------------------------------------------------------------------
 // Page means: kmean[b,h,j,d] = dtype(sum_t K[b,h,row0+j*page+t,d] / page).
 // One workgroup per (b, h, page).  Thread t owns the 16-byte piece
@@ -82,7 +93,9 @@ __global__ void __launch_bounds__(256) chunk_means_kernel(const void* k, int64_t
     const int c = d / EPC, e = d % EPC;
     float sum = 0.f;
     for (int g = 0; g < RG; ++g) sum += s_part[(g * SL + c) * 8 + e];
-    store_elem(km, (int64_t)b * msb + (int64_t)h * msh + (int64_t)j * msp + d, DT, sum * inv);
+    const int64_t o = (int64_t)b * msb + (int64_t)h * msh + (int64_t)j * msp + d;
+    if constexpr (DT == HALO_F16) reinterpret_cast<uint16_t*>(km)[o] = (uint16_t)mean_f16(sum, 0.f, inv);
+    else store_elem(km, o, DT, sum * inv);
   }
 }
 
@@ -128,16 +141,9 @@ __global__ void __launch_bounds__(256) chunk_means_col_kernel(const void* k, int
   const float inv = 1.0f / (float)page;
   const int64_t o = (int64_t)b * msb + (int64_t)h * msh + (int64_t)j * msp + col * EPC;
   if constexpr (DT == HALO_F16) {
-    // The other kernel's product and conversion are one v_fma_mixlo_f16, which
-    // rounds once; written out here so that both give the same bits.
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint32_t r = 0;
-      asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "+v"(r) : "v"(sum[2 * e]), "v"(inv));
-      asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(r) : "v"(sum[2 * e + 1]), "v"(inv));
-      w[e] = r;
-    }
+    for (int e = 0; e < 4; ++e) w[e] = mean_f16(sum[2 * e], sum[2 * e + 1], inv);
     uint16_t* dst = reinterpret_cast<uint16_t*>(km) + o;
     if (vec) {
       *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
