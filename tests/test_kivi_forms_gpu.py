@@ -30,6 +30,18 @@ def _inputs(dtype, D, n):
     return k, v
 
 
+def _zeros_positive(blocks, D, bits):
+    """Blocks (..., bytes) with -0 as +0 in the zeros of K and V (2D bytes each
+    behind the side's codes and scales)."""
+    out = blocks.copy()
+    codes = 32 * D * bits // 8
+    for end in (codes + 4 * D, 2 * codes + 8 * D):
+        z = np.ascontiguousarray(out[..., end - 2 * D:end]).view(np.uint16)
+        z[z == 0x8000] = 0
+        out[..., end - 2 * D:end] = z.view(np.uint8)
+    return out
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("D,n", [(64, 5), (128, 5), (256, 4)])
 @pytest.mark.parametrize("bits", [2, 4, 8])
@@ -40,9 +52,12 @@ def test_quantise_and_dequantise_forms(dev, dtype, D, n, bits):
     blocks = kivi.quantize(kt, vt, bits=bits)
     want = K.pack_blocks(k, v, bits=bits, dtype=dtype)
     got = blocks.cpu().numpy()
-    # the sign of a zero minimum is not pinned: compare blocks without the signed zeros' run, all others whole
+    # the sign of a zero minimum is not pinned: block 3 holds the signed zeros
     assert np.array_equal(np.delete(got, 3, axis=2), np.delete(want, 3, axis=2))
+    assert np.array_equal(_zeros_positive(got[:, :, 3], D, bits), _zeros_positive(want[:, :, 3], D, bits))
     rk, rv = K.unpack_blocks(got, D=D, bits=bits, dtype=dtype)
+    wk, wv = K.unpack_blocks(want, D=D, bits=bits, dtype=dtype)
+    assert np.array_equal(rk, wk) and np.array_equal(rv, wv)  # 0 == -0
     kd, vd = kivi.dequantize(blocks, D=D, dtype=TDT[dtype], bits=bits)
     assert np.array_equal(kd.float().cpu().numpy(), rk)
     assert np.array_equal(vd.float().cpu().numpy(), rv)
