@@ -6,7 +6,7 @@ reference uses, against the float64 closed form:
   T_q > 1 attention, halo/chunked_prefill.py:99-191; decode likewise), so a
   cold-tier read that is not ordered after the peel's device-to-host copy
   reads stale host rows and fails;
-* fp32 T_q > 1 (the decode kernel's fp32 path) and bf16 (MFMA prefill);
+* fp32 and bf16 T_q > 1 (MFMA prefill);
 * scorer-driven placement (pages kept on the GPU out of position order,
   halo/kv_cache_chunked.py:416-457) with exact causal positions.
 """
@@ -80,7 +80,7 @@ def test_peel_then_attention_without_sync(dev, dtype, tol):
 
 def test_prefill_rows_ragged_batch_fp32(dev):
     """fp32 T_q > 1 for B = 2 with per-row query starts through
-    prefill_attention (decode-kernel fp32 path), LSE included."""
+    prefill_attention (fp32 matrix form), LSE included."""
     from halo_amd.decode import ChunkRef
     from halo_amd.prefill import prefill_attention
     rng = np.random.default_rng(3)

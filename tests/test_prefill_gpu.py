@@ -69,9 +69,10 @@ def test_prefill_chunk_order_and_partition_invariance(dev):
     assert (la - lb).abs().max().item() <= 1e-3
 
 
-def test_prefill_fp32_runs_on_the_decode_path(dev):
+def test_prefill_fp32(dev):
     """fp32 queries are accepted (the reference computes any T_q in fp32,
-    halo/kv_cache_chunked.py:241-276) and match the float64 closed form."""
+    halo/kv_cache_chunked.py:241-276) and match the float64 closed form: two
+    causal chunks on the fp32 matrix form."""
     from halo_amd.decode import ChunkRef
     from halo_amd.prefill import prefill_attention
     rng = np.random.default_rng(21)
@@ -111,3 +112,32 @@ def test_prefill_on_a_side_stream(dev, dtype):
     want, wl = A.prefill_f64(q, k, v, scale=1 / 8, q_start=64)
     assert np.abs(out.float().cpu().numpy() - want).max() <= (1e-5 if dtype == "float32" else 2e-2)
     assert np.abs(lse.cpu().numpy() - wl).max() <= 1e-5 * max(1.0, np.abs(wl).max())
+
+
+@pytest.mark.parametrize("starts", ["per row", "number"])
+@pytest.mark.parametrize("T_prior,T_q,H,H_kv", [(70, 19, 6, 2), (0, 33, 4, 4), (300, 1, 8, 1)])
+def test_prefill_fp32_row_form(dev, starts, T_prior, T_q, H, H_kv):
+    """The row-by-row fp32 form (one decode launch per batch row), here for
+    chunk objects with just k, v, chunk_start and causal: query starts per
+    batch row, the LSE, and the refusals it keeps."""
+    from types import SimpleNamespace
+
+    from halo_amd.prefill import _f32_direct, prefill_attention
+    rng = np.random.default_rng(33)
+    B, D, T = 2, 64, T_prior + T_q
+    q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((B, H, T_q, D), (B, H_kv, T, D), (B, H_kv, T, D)))
+    qt, kt, vt = (torch.from_numpy(a).to(dev) for a in (q, k, v))
+    chunks = [SimpleNamespace(k=kt[:, :, a:a + 64], v=vt[:, :, a:a + 64], chunk_start=a, causal=True)
+              for a in range(0, T, 64)]
+    assert not _f32_direct(qt, chunks)
+    q0 = [T_prior, max(T_prior - 3, 0)] if starts == "per row" else [T_prior] * B
+    out, lse = prefill_attention(qt, chunks, return_lse=True,
+                                 q_start=torch.tensor(q0, device=dev) if starts == "per row" else T_prior)
+    for b in range(B):
+        want, wl = A.prefill_f64(q[b:b + 1], k[b:b + 1], v[b:b + 1], scale=1 / math.sqrt(D), q_start=q0[b])
+        assert np.abs(out[b:b + 1].cpu().numpy() - want).max() <= 1e-5
+        assert np.abs(lse[b:b + 1].cpu().numpy() - wl).max() <= 1e-5 * max(1.0, np.abs(wl).max())
+    off = torch.zeros(kt.numel() + 2, device=dev)[2:].view(kt.shape)
+    for odd in (off, torch.zeros((B, H_kv, T, D + 2), device=dev)[..., :D]):  # rows off 16 bytes
+        with pytest.raises(AssertionError, match="16-byte aligned"):
+            prefill_attention(qt, [SimpleNamespace(k=odd, v=odd, chunk_start=0, causal=True)], q_start=T_prior)
