@@ -46,7 +46,8 @@ extern "C" {
  * batch dimension (row b of the call's batch at k + b*k_stride_b); batch >= 0
  * means the chunk belongs to that batch row only (ragged / varlen tables) and
  * k points at that row's (h=0, t=0, d=0) element.  The head dimension is
- * contiguous (unit stride).  Replaces the (k, v, chunk_start, apply_causal)
+ * contiguous (unit stride) and rows do not overlap: reads end T_c row strides
+ * behind the first row.  Replaces the (k, v, chunk_start, apply_causal)
  * tuple of halo/triton_chunked.py:212 and the per-launch arguments of
  * halo/triton_chunked.py:180-192.
  */
