@@ -266,12 +266,12 @@ __device__ __forceinline__ void kivi_store_codes(const uint16_t* s_k, const uint
 // column and row-run reads spread over the banks); 512/D threads reduce each
 // pair of K channels and two each V (token, 32-channel group) to its min / max;
 // then each thread codes 8 channels of D/64 output rows (K, token-major) and
-// two channels x 8 slots (V, channel-major in slot order) and stores packed
-// bytes.  An element costs about 14 VALU operations (bf16 rounding in hardware
+// two channels x 8 slots (V, channel-major in slot order), at D = 64 one of the
+// two with as much work, and stores packed bytes.  An element costs about 14 VALU operations (bf16 rounding in hardware
 // two at a time, no per-element range branch, codes packed by fp32
 // multiply-adds of up to 16 bits), where rounding by hand and a checked quotient
 // took 23 in fp16 and more than twice that in bf16.  32768 tokens x 8 heads x 128
-// bf16 in 2 bits: 102.9 us before, 46.2 now (3.4 TB/s), bound by the phases
+// bf16 in 2 bits: 102.9 us before, 45.7 now (3.4 TB/s), bound by the phases
 // behind its barriers.  Workgroups that walk several blocks with the next
 // block's loads in flight took 69: the barriers wait for those loads.
 template <int DT, int D, int BITS>

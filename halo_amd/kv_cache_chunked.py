@@ -29,8 +29,8 @@ What changes on MI355X:
     staging buffers merged into fp32 accumulators, and
     ``HALO_TRITON_SINGLE_LAUNCH=1`` stages the whole cold tier in HBM first
     and attends it with the GPU rows in one launch.  T_q > 1 stages the cold
-    chunks and runs one ``halo_prefill_attn`` (bf16/fp16 MFMA; fp32 on the
-    decode kernel's fp32 path) over them and the GPU rows;
+    chunks and runs one ``halo_prefill_attn_split`` (MFMA in bf16, fp16 and
+    fp32) over them and the GPU rows;
   * per-chunk fp32 key sums are accumulated at peel time, so every filled
     cold chunk has its mean key on the GPU (the page-mean metadata a chunk
     scorer reads) without touching host memory.
@@ -218,8 +218,7 @@ class HALOCacheChunked(HALOCache):
         """Attention of q (B, H, T_q, D) over one chunk (B, H_kv, T_c, D),
         query heads grouped over the KV heads, returning the fp32 partial
         (out (B, H, T_q, D), lse (B, H, T_q)) (halo/kv_cache_chunked.py:
-        241-276): one prefill launch (``halo_prefill_attn``; fp32 through the
-        decode kernel).  The kernels mask by position, so ``causal_mask``
+        241-276): one prefill call (``halo_prefill_attn_split``).  The kernels mask by position, so ``causal_mask``
         (T_q, T_c, additive) is taken in the form the reference's chunk walk
         builds -- 0 where key j <= q_start + i, -inf elsewhere, for some
         offset q_start -- and any other mask raises."""
